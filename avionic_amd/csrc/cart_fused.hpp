@@ -23,17 +23,6 @@ constexpr int NTC = AVIONIC_COL_THREADS;  // threads of a column-pass block
 // Outputs per lane of a column-pass stage (narrow / wide plans).
 constexpr int col_slots(bool wide) { return max_slots(kColTileElems, NTC, wide); }
 
-// (i + n/2) mod n and (a + b) mod n for 0 <= i, a < n, 0 <= b <= n, without a
-// division.
-__device__ __forceinline__ int wrap_half(int i, int n) {
-  const int v = i + n / 2;
-  return v >= n ? v - n : v;
-}
-__device__ __forceinline__ int wrap_add(int a, int b, int n) {
-  const int v = a + b;
-  return v >= n ? v - n : v;
-}
-
 // ------------------------------------------------------------ column plans
 // A column pass runs on the geometry's runtime plan (g.ph, g.XBF) or on one
 // of a few compile-time plans.  With a compile-time plan every index of the
@@ -281,9 +270,9 @@ __device__ inline const int *stage_rowmap(const CartGeom &g, int t, int *lds, in
 }
 
 template <bool DELTA, class P>
-__device__ inline void col_forward_fused(const CartGeom &g, int xbi, int t, const float2 *u,
-                                         const float2 *usub, const float2 *b1, float2 *kcol,
-                                         float2 *tile, float2 *twl, int *rml) {
+__device__ inline void col_forward_fused(const CartGeom &g, int xbi, int t, int c0, int c1,
+                                         const float2 *u, const float2 *usub, const float2 *b1,
+                                         float2 *kcol, float2 *tile, float2 *twl, int *rml) {
   const int tid = threadIdx.x;
   const long HW = (long)g.H * g.W;
   const int XB = P::XB ? P::XB : g.XBF;
@@ -299,8 +288,8 @@ __device__ inline void col_forward_fused(const CartGeom &g, int xbi, int t, cons
   ld.xb0 = xbi * XB;
   ld.centered = g.centered;
   ColFwdStore<P::H> st{nullptr, rmap, g.H, g.W, xbi * XB, g.centered};
-  for (int c = 0; c < g.C; ++c) {
-    ld.first = c == 0;
+  for (int c = c0; c < c1; ++c) {
+    ld.first = c == c0;
     ld.bc = b1 + c * HW;
     st.kc = kcol + ((long)g.C * r0 + (long)c * S) * g.W;
     if constexpr (P::H == 0)
@@ -461,6 +450,51 @@ struct RowNorm2Store {
     const int kx = centered ? wrap_half(i, W) : i;
     const float2 val = cscale(v, scale * gld(mrows, (unsigned)(mrow[b] * W + kx)));
     acc += (double)cabs2(val);
+  }
+};
+// |K u - d|^2 on the compact data
+struct RowResidualStore {
+  const float *mrows;
+  const int *mrow;
+  const float2 *d;  // d + g0 W
+  int W, centered;
+  float scale;
+  double acc;
+  __device__ void operator()(int b, int i, float2 v, int) {
+    const int kx = centered ? wrap_half(i, W) : i;
+    const float2 val = cscale(v, scale * gld(mrows, (unsigned)(mrow[b] * W + kx)));
+    acc += (double)cabs2(csub(val, gld(d, (unsigned)(b * W + kx))));
+  }
+};
+// K u into the dense k-space
+struct RowApplyStore {
+  const float *mrows;
+  const int *mrow;
+  const int4 *info;  // rowinfo + g0
+  float2 *out;
+  int W, C, H, centered;
+  float scale;
+  __device__ void operator()(int b, int i, float2 v, int) {
+    const int kx = centered ? wrap_half(i, W) : i;
+    const int4 ri = info[b];
+    out[(((long)ri.x * C + ri.y) * H + ri.w) * W + kx] =
+        cscale(v, scale * gld(mrows, (unsigned)(mrow[b] * W + kx)));
+  }
+};
+// M z of dense or compact k-space
+template <bool DENSE>
+struct RowMaskLoad {
+  const float *mrows;
+  const int *mrow;
+  const int4 *info;
+  const float2 *z;  // dense: the whole k-space; compact: z + g0 W
+  int W, C, H, centered;
+  __device__ float2 operator()(int b, int i, int) const {
+    const int kx = centered ? wrap_half(i, W) : i;
+    const float mk = gld(mrows, (unsigned)(mrow[b] * W + kx));
+    if (!DENSE) return cscale(gld(z, (unsigned)(b * W + kx)), mk);
+    const int4 ri = info[b];
+    return cscale(z[(((long)ri.x * C + ri.y) * H + ri.w) * W + kx], mk);
   }
 };
 
@@ -695,9 +729,12 @@ __device__ inline double row_fused_ct(const CartGeom &g, int blk, const float2 *
   return 0.0;
 }
 
-template <bool WIDE>
-__device__ inline double row_norm2_fused(const CartGeom &g, int blk, const float2 *kcol,
-                                         float2 *tile, float2 *twl, int *mrl) {
+// The modes other than the dual update on a runtime plan; returns the lane's
+// part of the sum (kRowNorm2, kRowResidual).
+template <int MODE, bool WIDE>
+__device__ inline double row_mode_fused(const CartGeom &g, int blk, const float2 *kcol,
+                                        const float2 *d, float2 *zhat, float2 *out,
+                                        const float2 *zin, float2 *tile, float2 *twl, int *mrl) {
   const int tid = threadIdx.x;
   const int W = g.W;
   const long g0 = (long)blk * g.RB;
@@ -705,10 +742,29 @@ __device__ inline double row_norm2_fused(const CartGeom &g, int blk, const float
   const float2 *tw = stage_twiddles(g.pw, twl, tid, NT);
   const int *mrow = stage_mask_rows(g, g0, nr, mrl, tid, NT);
   __syncthreads();
-  RowLoad ld{kcol + g0 * W, W};
-  RowNorm2Store st{g.mrows, mrow, W, g.centered, g.scale, 0.0};
-  fft_io<NT, RTILE, false, true, true, WIDE>(tile, g.pw, nr, W, 1, +1.f, tid, tw, ld, st);
-  return st.acc;
+  if constexpr (MODE == kRowAdjDense || MODE == kRowAdjCompact) {
+    constexpr bool DENSE = MODE == kRowAdjDense;
+    RowMaskLoad<DENSE> ld{g.mrows, mrow, g.rowinfo + g0, DENSE ? zin : zin + g0 * W,
+                          W, g.C, g.H, g.centered};
+    RowAdjStore st{zhat + g0 * W, W, g.centered};
+    fft_io<NT, RTILE, false, true, true, WIDE>(tile, g.pw, nr, W, 1, -1.f, tid, tw, ld, st);
+    return 0.0;
+  } else {
+    RowLoad ld{kcol + g0 * W, W};
+    if constexpr (MODE == kRowApplyK) {
+      RowApplyStore st{g.mrows, mrow, g.rowinfo + g0, out, W, g.C, g.H, g.centered, g.scale};
+      fft_io<NT, RTILE, false, true, true, WIDE>(tile, g.pw, nr, W, 1, +1.f, tid, tw, ld, st);
+      return 0.0;
+    } else if constexpr (MODE == kRowNorm2) {
+      RowNorm2Store st{g.mrows, mrow, W, g.centered, g.scale, 0.0};
+      fft_io<NT, RTILE, false, true, true, WIDE>(tile, g.pw, nr, W, 1, +1.f, tid, tw, ld, st);
+      return st.acc;
+    } else {
+      RowResidualStore st{g.mrows, mrow, d + g0 * W, W, g.centered, g.scale, 0.0};
+      fft_io<NT, RTILE, false, true, true, WIDE>(tile, g.pw, nr, W, 1, +1.f, tid, tw, ld, st);
+      return st.acc;
+    }
+  }
 }
 
 }  // namespace avionic

@@ -22,9 +22,10 @@ namespace avionic {
 struct CartGeom {
   int W, H, C, T;
   int centered;
-  int XB;  // columns per column-pass tile (API kernels)
-  int RB;  // rows per row-pass tile
-  int nxb;
+  int RB;  // rows per row-pass block on a runtime plan
+  // Two-stage passes (cart_two.hpp), where the length has radices ra, rb:
+  int XB, lxb, nxb;  // columns per tile (2^lxb), tiles
+  int RBT, ljw;      // rows per row-pass block, NT / 2^ljw
   int XBF, nxbf;  // columns per tile / tiles of the hot loop's fused column passes
   int cplan;      // compile-time plan of the fused column passes (ColPlanId)
   int rplan;      // compile-time plan of the fused row pass (RowPlanId)
@@ -60,7 +61,7 @@ __host__ __device__ inline int row_kind(const CartGeom &g) {
 }
 
 // Row-pass modes.
-enum RowMode {
+enum RowMode {  // Norm2, Residual: RBT (two-stage) or RB rows per partial sum
   kRowApplyK = 0,     // out = K(u) rows (compact or dense)
   kRowDualUpdate = 1, // z = (z + s K u - s d)/(1 + s/l); zhat = F_row(M z)
   kRowNorm2 = 2,      // partial sums of |K u|^2
@@ -88,7 +89,10 @@ struct CartPlan {
   // mask: device pointer [T][H][W] or nullptr.
   void init(int W, int H, int C, int T, const float *mask, int centered, hipStream_t s);
   long kspace_elems() const { return g.nrows_c * (long)g.W; }
-  int row_blocks() const { return (int)((g.nrows_c + g.RB - 1) / g.RB); }
+  int row_blocks() const {
+    const int rb = g.pw.ra ? g.RBT : g.RB;
+    return (int)((g.nrows_c + rb - 1) / rb);
+  }
   int fused_row_blocks() const { return (int)((g.nrows_c + g.RBF - 1) / g.RBF); }
 };
 

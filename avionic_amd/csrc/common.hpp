@@ -296,6 +296,7 @@ struct FftPlan {
   int nst;
   int radix[kMaxStages];
   int ns[kMaxStages];
+  int ra, rb;        // L = ra rb with 16 >= ra >= rb (0: no such pair)
   const float2 *tw;  // tw[m] = exp(-2 pi i m / L), m < L (device)
 };
 __host__ __device__ inline bool plan_is_wide(const FftPlan &p) {

@@ -149,6 +149,94 @@ struct Dft<16> {
   }
 };
 
+template <>
+struct Dft<1> {
+  __device__ static inline void run(float2 *, float) {}
+};
+
+// Composite radix N = P Q, P and Q coprime, by the prime-factor mapping:
+// inputs at (Q n1 + P n2) mod N, outputs at the k with k = k1 mod P and
+// k = k2 mod Q, so that no twiddles stand between the two factors.
+template <int P, int Q>
+struct DftPfa {
+  static constexpr int N = P * Q;
+  __host__ __device__ static constexpr int out_index(int k1, int k2) {
+    for (int k = 0; k < N; ++k)
+      if (k % P == k1 && k % Q == k2) return k;
+    return 0;
+  }
+  __device__ static inline void run(float2 *v, float sign) {
+    float2 a[Q][P];
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) {
+#pragma unroll
+      for (int n1 = 0; n1 < P; ++n1) a[n2][n1] = v[(Q * n1 + P * n2) % N];
+      Dft<P>::run(a[n2], sign);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) {
+      float2 b[Q];
+#pragma unroll
+      for (int n2 = 0; n2 < Q; ++n2) b[n2] = a[n2][k1];
+      Dft<Q>::run(b, sign);
+#pragma unroll
+      for (int k2 = 0; k2 < Q; ++k2) v[out_index(k1, k2)] = b[k2];
+    }
+  }
+};
+template <> struct Dft<6> : DftPfa<2, 3> {};
+template <> struct Dft<10> : DftPfa<2, 5> {};
+template <> struct Dft<12> : DftPfa<4, 3> {};
+template <> struct Dft<14> : DftPfa<2, 7> {};
+template <> struct Dft<15> : DftPfa<3, 5> {};
+
+template <>
+struct Dft<9> {
+  // 3 x 3: n = 3 n1 + n2, k = k1 + 3 k2, twiddles w9^(n2 k1) between.
+  __device__ static inline void run(float2 *v, float sign) {
+    float2 a[3][3];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+      a[n2][0] = v[n2]; a[n2][1] = v[3 + n2]; a[n2][2] = v[6 + n2];
+      Dft<3>::run(a[n2], sign);
+    }
+    a[1][1] = crot(a[1][1], 0.76604444311897801f, 0.64278760968653925f, sign);
+    a[1][2] = crot(a[1][2], 0.17364817766693041f, 0.98480775301220802f, sign);
+    a[2][1] = crot(a[2][1], 0.17364817766693041f, 0.98480775301220802f, sign);
+    a[2][2] = crot(a[2][2], -0.93969262078590832f, 0.34202014332566888f, sign);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      float2 b[3] = {a[0][k1], a[1][k1], a[2][k1]};
+      Dft<3>::run(b, sign);
+      v[k1] = b[0]; v[k1 + 3] = b[1]; v[k1 + 6] = b[2];
+    }
+  }
+};
+
+// Calls f(std::integral_constant<int, R>) for a runtime radix 1 .. kMaxRadix.
+constexpr int kMaxRadix = 16;
+template <class F>
+__device__ __forceinline__ void with_radix(int R, F &&f) {
+  switch (R) {
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    case 15: f(std::integral_constant<int, 15>{}); break;
+    case 14: f(std::integral_constant<int, 14>{}); break;
+    case 13: f(std::integral_constant<int, 13>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 11: f(std::integral_constant<int, 11>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, 1>{}); break;
+  }
+}
+
 // One Stockham stage.  Must be called by all NT threads of the block.
 // BFAST: consecutive lanes take consecutive transforms (b) instead of
 // consecutive butterflies (j); pick the one whose LDS stride is 1.

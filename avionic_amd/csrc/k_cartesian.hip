@@ -1,5 +1,5 @@
-// Cartesian operator kernels for the per-operator API (K, K^H, norms); the
-// block bodies live in cart_device.hpp.
+// Cartesian plans, the compact gather and the standalone 2D transform; the
+// operator's column and row passes are in k_cart_col.hip and k_cart_row.hip.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -7,37 +7,6 @@
 #include "cart_device.hpp"
 
 namespace avionic {
-
-__global__ __launch_bounds__(NT) void k_col_forward(CartGeom g, const float2 *__restrict__ u,
-                                                    const float2 *__restrict__ usub,
-                                                    const float2 *__restrict__ b1,
-                                                    float2 *__restrict__ kcol) {
-  __shared__ float2 tile[EMAX];
-  col_forward_block(g, blockIdx.x, blockIdx.y, u, usub, b1, kcol, tile);
-}
-
-template <int MODE>
-__global__ __launch_bounds__(NT) void k_row_pass(CartGeom g, const float2 *__restrict__ kcol,
-                                                 float2 *__restrict__ z,
-                                                 const float2 *__restrict__ d,
-                                                 float2 *__restrict__ zhat,
-                                                 float2 *__restrict__ out,
-                                                 const float2 *__restrict__ zin,
-                                                 const DevScalars *__restrict__ sc,
-                                                 double *__restrict__ partial) {
-  __shared__ float2 tile[EMAX];
-  __shared__ float2 tile2[(MODE == kRowDualUpdate) ? EMAX : 1];
-  __shared__ double red[NT];
-  row_pass_block<MODE>(g, blockIdx.x, kcol, z, d, zhat, out, zin, sc, partial, tile, tile2, red);
-}
-
-__global__ __launch_bounds__(NT) void k_col_adjoint(CartGeom g, const float2 *__restrict__ zhat,
-                                                    const float2 *__restrict__ b1,
-                                                    float2 *__restrict__ out) {
-  __shared__ float2 tile[EMAX];
-  __shared__ float2 acc[EMAX];
-  col_adjoint_block(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile, acc);
-}
 
 // Dense [t][c][H][W] -> compact rows, times the mask.
 __global__ void k_compact_gather(CartGeom g, const float2 *__restrict__ dense,
@@ -115,6 +84,17 @@ static int pick_xb(int H, int W, int emax = EMAX) {
   return xb;
 }
 
+// Radices of a two-stage transform: the pair closest to square (fewest idle
+// lanes), the larger first.
+static void pick_two_stage(FftPlan &p) {
+  for (int rb = kMaxRadix; rb >= 1; --rb)
+    if (rb * rb <= p.L && p.L % rb == 0 && p.L / rb <= kMaxRadix) {
+      p.ra = p.L / rb;
+      p.rb = rb;
+      return;
+    }
+}
+
 static int pick_col_plan(int H, int XBF) {
   if (H == 256 && XBF == 16) return kColPlan256;
   if (H == 128 && XBF == 32) return kColPlan128;
@@ -141,6 +121,7 @@ void make_fft_plan(int L, FftPlan &p, void **d_tw) {
     }
   }
   AV_CHECK(m == 1, "FFT length must factor into 2, 3, 5, 7, 11 and 13");
+  pick_two_stage(p);
   std::vector<float2> tw(L);
   for (int k = 0; k < L; ++k) {
     const double a = -2.0 * M_PI * (double)k / (double)L;
@@ -163,9 +144,7 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   g = CartGeom{};
   g.W = W; g.H = H; g.C = C; g.T = T;
   g.centered = centered ? 1 : 0;
-  g.XB = pick_xb(H, W);
   g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / W));
-  g.nxb = (W + g.XB - 1) / g.XB;
   g.XBF = pick_xb(H, W, kColTileElems);
   g.nxbf = (W + g.XBF - 1) / g.XBF;
   g.cplan = pick_col_plan(H, g.XBF);
@@ -228,6 +207,18 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   g.rowmap = (const int *)d_rowmap;
   make_fft_plan(W, g.pw, &d_twx);
   make_fft_plan(H, g.ph, &d_twy);
+  if (g.ph.ra) {
+    g.XB = 1;
+    while (g.XB * 2 * g.ph.ra <= NT && g.XB * 2 <= 64 && g.XB < W) {
+      g.XB *= 2;
+      g.lxb += 1;
+    }
+    g.nxb = (W + g.XB - 1) / g.XB;
+  }
+  if (g.pw.ra) {
+    while ((1 << g.ljw) < g.pw.ra) g.ljw += 1;
+    g.RBT = NT >> g.ljw;
+  }
   g.wide_col = plan_is_wide(g.ph) ? 1 : 0;
   g.wide_row = plan_is_wide(g.pw) ? 1 : 0;
   // The tables above come from pageable host memory: such a copy (on the
@@ -236,36 +227,6 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   // the null stream.  Waiting for the null stream alone leaves those streams'
   // own work running.
   AV_HIP(hipStreamSynchronize(nullptr));
-}
-
-void launch_col_forward(const CartGeom &g, const float2 *u, const float2 *usub, const float2 *b1,
-                        float2 *kcol, hipStream_t s) {
-  hipLaunchKernelGGL(k_col_forward, dim3(g.nxb, g.T), dim3(NT), 0, s, g, u, usub, b1, kcol);
-  AV_LAUNCH_CHECK();
-}
-
-void launch_row_pass(int mode, const CartGeom &g, const float2 *kcol, float2 *z, const float2 *d,
-                     float2 *zhat, float2 *out, const float2 *zin, const DevScalars *sc,
-                     double *partial, hipStream_t s) {
-  const int nb = (int)((g.nrows_c + g.RB - 1) / g.RB);
-  if (nb == 0) return;
-  dim3 grid(nb), block(NT);
-  switch (mode) {
-    case kRowApplyK: hipLaunchKernelGGL(k_row_pass<kRowApplyK>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRowDualUpdate: hipLaunchKernelGGL(k_row_pass<kRowDualUpdate>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRowNorm2: hipLaunchKernelGGL(k_row_pass<kRowNorm2>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRowAdjDense: hipLaunchKernelGGL(k_row_pass<kRowAdjDense>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRowResidual: hipLaunchKernelGGL(k_row_pass<kRowResidual>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRowAdjCompact: hipLaunchKernelGGL(k_row_pass<kRowAdjCompact>, grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    default: AV_CHECK(false, "bad row-pass mode");
-  }
-  AV_LAUNCH_CHECK();
-}
-
-void launch_col_adjoint(const CartGeom &g, const float2 *zhat, const float2 *b1, float2 *out,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_col_adjoint, dim3(g.nxb, g.T), dim3(NT), 0, s, g, zhat, b1, out);
-  AV_LAUNCH_CHECK();
 }
 
 void launch_compact_gather(const CartGeom &g, const float2 *dense, float2 *compact, hipStream_t s) {

@@ -112,7 +112,7 @@ template <bool DELTA, class P>
 __device__ __forceinline__ void col_forward_task(const Task &T, int lb, float2 *tile, float2 *twl,
                                                  int *rml) {
   const int xbi = lb % T.cg.nxbf, t = lb / T.cg.nxbf;
-  col_forward_fused<DELTA, P>(T.cg, xbi, t, T.ext, DELTA ? T.x : nullptr, T.b1, T.kcol, tile, twl,
+  col_forward_fused<DELTA, P>(T.cg, xbi, t, 0, T.cg.C, T.ext, DELTA ? T.x : nullptr, T.b1, T.kcol, tile, twl,
                               rml);
 }
 template <class P>
@@ -186,7 +186,8 @@ __global__ __launch_bounds__(NT) void kt_row(const Task *__restrict__ tasks, int
     if (MODE == kRowDualUpdate)
       row_dual_fused<RK == 2>(T.cg, lb, T.kcol, T.z, T.d, T.zhat, T.sc, tile, tile2, twl, mrl);
     else
-      a = row_norm2_fused<RK == 2>(T.cg, lb, T.kcol, tile, twl, mrl);
+      a = row_mode_fused<kRowNorm2, RK == 2>(T.cg, lb, T.kcol, nullptr, nullptr, nullptr, nullptr, tile,
+                                             twl, mrl);
   }
   if (MODE == kRowNorm2) {
     const int tid = threadIdx.x;
