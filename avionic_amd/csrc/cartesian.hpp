@@ -19,17 +19,16 @@
 
 namespace avionic {
 
+// Two-stage passes: butterflies of the radix-rb stage that one lane runs at
+// most (16 values in registers).
+__host__ __device__ constexpr int two_most(int rb) { return rb <= 4 ? 4 : (rb <= 8 ? 2 : 1); }
+
 struct CartGeom {
   int W, H, C, T;
   int centered;
-  int RB;  // rows per row-pass block on a runtime plan
-  // Two-stage passes (cart_two.hpp), where the length has radices ra, rb:
-  int XB, lxb, nxb;  // columns per tile (2^lxb), tiles
-  int RBT, ljw;      // rows per row-pass block, NT / 2^ljw
-  int XBF, nxbf;  // columns per tile / tiles of the hot loop's fused column passes
-  int cplan;      // compile-time plan of the fused column passes (ColPlanId)
-  int rplan;      // compile-time plan of the fused row pass (RowPlanId)
-  int RBF;        // rows per block of the fused row pass
+  int XB, lxb, nxb;  // columns per column-pass tile (two-stage: 2^lxb), tiles
+  int RB;            // rows per row-pass block
+  int lja, ljb;      // two-stage: log2 of the lanes per row in the radix-ra / -rb stages
   int wide_col, wide_row;  // column / row plan is wide (plan_is_wide)
   long nrows;          // sampled rows over all frames (row_off[T])
   long nrows_c;        // C * nrows
@@ -42,26 +41,20 @@ struct CartGeom {
   FftPlan pw, ph;
 };
 
-// Compile-time column plans (transform length H, XBF columns per tile); any
-// other geometry runs the runtime plan.
-enum ColPlanId { kColPlanRt = 0, kColPlan256, kColPlan128, kColPlan160, kColPlan192, kColPlan224 };
-// Kind of a geometry's fused column passes: 0 runtime plan, 1 compile-time
-// plan, 2 wide runtime plan (one kernel per kind).
-constexpr int kColKinds = 3;
+// Kind of a geometry's column passes (one kernel per kind): 0 runtime plan,
+// 1 two-stage (cart_two.hpp), 2 wide runtime plan, 3 two-stage, length 256.
+constexpr int kColKinds = 4;
 __host__ __device__ inline int col_kind(const CartGeom &g) {
-  return g.cplan != kColPlanRt ? 1 : (g.wide_col ? 2 : 0);
+  return g.ph.ra ? (g.ph.L == 256 && g.lxb == 4 ? 3 : 1) : (g.wide_col ? 2 : 0);
 }
-// Compile-time row plans (row length W); rows per block 16 and 32.
-enum RowPlanId { kRowPlanRt = 0, kRowPlan256, kRowPlan128 };
-// Kind of the fused row pass: 0 compile-time plan, 1 runtime plan, 2 wide
-// runtime plan (one kernel per kind).
+// Kind of the row pass: 0 two-stage, 1 runtime plan, 2 wide runtime plan.
 constexpr int kRowKinds = 3;
 __host__ __device__ inline int row_kind(const CartGeom &g) {
-  return g.rplan != kRowPlanRt ? 0 : (g.wide_row ? 2 : 1);
+  return g.pw.ra ? 0 : (g.wide_row ? 2 : 1);
 }
 
 // Row-pass modes.
-enum RowMode {  // Norm2, Residual: RBT (two-stage) or RB rows per partial sum
+enum RowMode {  // Norm2, Residual: one partial sum per row block
   kRowApplyK = 0,     // out = K(u) rows (compact or dense)
   kRowDualUpdate = 1, // z = (z + s K u - s d)/(1 + s/l); zhat = F_row(M z)
   kRowNorm2 = 2,      // partial sums of |K u|^2
@@ -89,12 +82,17 @@ struct CartPlan {
   // mask: device pointer [T][H][W] or nullptr.
   void init(int W, int H, int C, int T, const float *mask, int centered, hipStream_t s);
   long kspace_elems() const { return g.nrows_c * (long)g.W; }
-  int row_blocks() const {
-    const int rb = g.pw.ra ? g.RBT : g.RB;
-    return (int)((g.nrows_c + rb - 1) / rb);
-  }
-  int fused_row_blocks() const { return (int)((g.nrows_c + g.RBF - 1) / g.RBF); }
+  int row_blocks() const { return (int)((g.nrows_c + g.RB - 1) / g.RB); }
 };
+
+// Column tiles of a geometry's two-stage passes.  Wide tiles keep every lane
+// busy in both stages; narrow ones give more blocks.  The results do not depend
+// on the choice.
+void set_col_tiles(CartGeom &g, bool wide);
+// Blocks of a column pass on wide tiles, and the count from which wide tiles
+// are taken: two blocks per CU.
+long wide_col_blocks(const CartGeom &g);
+constexpr long kColWideBlocks = 512;
 
 void make_fft_plan(int L, FftPlan &p, void **d_tw);
 

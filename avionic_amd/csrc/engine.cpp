@@ -203,6 +203,15 @@ struct avionic_engine {
       const int ka = col_kind(a->task.cg), kb = col_kind(b->task.cg);
       return ka != kb ? ka < kb : row_kind(a->task.cg) < row_kind(b->task.cg);
     });
+    // column tiles by the launch set's size (the results do not depend on them)
+    long wide = 0;
+    for (const Slot *s : g.slots)
+      if (s->cart) wide += wide_col_blocks(s->task.cg);
+    for (Slot *s : g.slots)
+      if (s->cart) {
+        set_col_tiles(s->task.cg, wide >= kColWideBlocks);
+        s->task.ncol_blocks = s->task.cg.nxb * s->task.cg.T;
+      }
     std::vector<Task> tasks;
     int bv = 0, bd1 = 0, bd2 = 0, bc = 0, br = 0;
     g.grid = TaskGrid{};
@@ -578,7 +587,7 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
     s->tlog.ensure(sizeof(double) * std::max(1, s->maxit));
     const Grid3 g{s->W, s->H, s->T, N};
     const int nvb = step_blocks(g);
-    const int nrb = s->cart ? s->cart->plan().fused_row_blocks() : 0;
+    const int nrb = s->cart ? s->cart->plan().row_blocks() : 0;
     const int npk = s->cart ? nrb : s->op->max_partials();
     s->preg.ensure(sizeof(double) * 2 * nvb);
     s->pk.ensure(sizeof(double) * std::max(1, npk));
@@ -643,7 +652,7 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
     const bool pairs = g.W % 2 == 0;
     t.ndp1_blocks = pairs ? 0 : nvb;
     t.ndp2_blocks = pairs ? pair_blocks(g) : 0;
-    t.ncol_blocks = s->cart ? t.cg.nxbf * t.cg.T : 0;
+    t.ncol_blocks = s->cart ? t.cg.nxb * t.cg.T : 0;
     t.nrow_blocks = nrb;
     t.npart_k = npk;
     t.schedule = s->params.adaptSchedule;

@@ -10,13 +10,15 @@ __global__ __launch_bounds__(NT) void k_col_forward(CartGeom g, const float2 *__
                                                     const float2 *__restrict__ usub,
                                                     const float2 *__restrict__ b1,
                                                     float2 *__restrict__ kcol) {
-  __shared__ float2 tile[KIND == kTwo ? kColTwoElems : kColTileElems];
-  __shared__ float2 twl[api_table_len(KIND)];
-  __shared__ int rml[api_table_len(KIND)];
-  if constexpr (KIND == kTwo)
-    col_forward_two<DELTA>(g, blockIdx.x, blockIdx.y, 0, g.C, u, usub, b1, kcol, tile, twl, rml);
+  __shared__ float2 tile[KIND & 1 ? kColTwoElems : kColTileElems];
+  __shared__ float2 twl[col_table_len(KIND)];
+  __shared__ int rml[col_table_len(KIND)];
+  if constexpr (KIND == 1)
+    col_forward_two<DELTA, TwoRt>(g, blockIdx.x, blockIdx.y, 0, g.C, u, usub, b1, kcol, tile, twl, rml);
+  else if constexpr (KIND == 3)
+    col_forward_two<DELTA, Two256>(g, blockIdx.x, blockIdx.y, 0, g.C, u, usub, b1, kcol, tile, twl, rml);
   else
-    col_forward_fused<DELTA, ColPlanRtT<KIND == kRtWide>>(g, blockIdx.x, blockIdx.y, 0, g.C, u,
+    col_forward_fused<DELTA, KIND == 2>(g, blockIdx.x, blockIdx.y, 0, g.C, u,
                                                           usub, b1, kcol, tile, twl, rml);
 }
 
@@ -24,24 +26,27 @@ template <int KIND>
 __global__ __launch_bounds__(NT) void k_col_adjoint(CartGeom g, const float2 *__restrict__ zhat,
                                                     const float2 *__restrict__ b1,
                                                     float2 *__restrict__ out) {
-  __shared__ float2 tile[KIND == kTwo ? kColTwoElems : kColTileElems];
-  __shared__ float2 twl[api_table_len(KIND)];
-  __shared__ int rml[api_table_len(KIND)];
-  if constexpr (KIND == kTwo)
-    col_adjoint_two(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile, twl, rml);
+  __shared__ float2 tile[KIND & 1 ? kColTwoElems : kColTileElems];
+  __shared__ float2 twl[col_table_len(KIND)];
+  __shared__ int rml[col_table_len(KIND)];
+  if constexpr (KIND == 1)
+    col_adjoint_two<TwoRt>(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile, twl, rml);
+  else if constexpr (KIND == 3)
+    col_adjoint_two<Two256>(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile, twl, rml);
   else
-    col_adjoint_fused<ColPlanRtT<KIND == kRtWide>>(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile,
+    col_adjoint_fused<KIND == 2>(g, blockIdx.x, blockIdx.y, zhat, b1, out, tile,
                                                    twl, rml);
 }
 
 template <bool DELTA>
 static void launch_col_fwd_kind(const CartGeom &g, const float2 *u, const float2 *usub,
                                 const float2 *b1, float2 *kcol, hipStream_t s) {
-  const dim3 two(g.nxb, g.T), rt(g.nxbf, g.T), block(NT);
-  switch (api_kind(g.ph)) {
-    case kTwo: hipLaunchKernelGGL((k_col_forward<DELTA, kTwo>), two, block, 0, s, g, u, usub, b1, kcol); break;
-    case kRt: hipLaunchKernelGGL((k_col_forward<DELTA, kRt>), rt, block, 0, s, g, u, usub, b1, kcol); break;
-    default: hipLaunchKernelGGL((k_col_forward<DELTA, kRtWide>), rt, block, 0, s, g, u, usub, b1, kcol); break;
+  const dim3 grid(g.nxb, g.T), block(NT);
+  switch (col_kind(g)) {
+    case 1: hipLaunchKernelGGL((k_col_forward<DELTA, 1>), grid, block, 0, s, g, u, usub, b1, kcol); break;
+    case 0: hipLaunchKernelGGL((k_col_forward<DELTA, 0>), grid, block, 0, s, g, u, usub, b1, kcol); break;
+    case 3: hipLaunchKernelGGL((k_col_forward<DELTA, 3>), grid, block, 0, s, g, u, usub, b1, kcol); break;
+    default: hipLaunchKernelGGL((k_col_forward<DELTA, 2>), grid, block, 0, s, g, u, usub, b1, kcol); break;
   }
   AV_LAUNCH_CHECK();
 }
@@ -56,11 +61,12 @@ void launch_col_forward(const CartGeom &g, const float2 *u, const float2 *usub, 
 
 void launch_col_adjoint(const CartGeom &g, const float2 *zhat, const float2 *b1, float2 *out,
                         hipStream_t s) {
-  const dim3 two(g.nxb, g.T), rt(g.nxbf, g.T), block(NT);
-  switch (api_kind(g.ph)) {
-    case kTwo: hipLaunchKernelGGL((k_col_adjoint<kTwo>), two, block, 0, s, g, zhat, b1, out); break;
-    case kRt: hipLaunchKernelGGL((k_col_adjoint<kRt>), rt, block, 0, s, g, zhat, b1, out); break;
-    default: hipLaunchKernelGGL((k_col_adjoint<kRtWide>), rt, block, 0, s, g, zhat, b1, out); break;
+  const dim3 grid(g.nxb, g.T), block(NT);
+  switch (col_kind(g)) {
+    case 1: hipLaunchKernelGGL((k_col_adjoint<1>), grid, block, 0, s, g, zhat, b1, out); break;
+    case 0: hipLaunchKernelGGL((k_col_adjoint<0>), grid, block, 0, s, g, zhat, b1, out); break;
+    case 3: hipLaunchKernelGGL((k_col_adjoint<3>), grid, block, 0, s, g, zhat, b1, out); break;
+    default: hipLaunchKernelGGL((k_col_adjoint<2>), grid, block, 0, s, g, zhat, b1, out); break;
   }
   AV_LAUNCH_CHECK();
 }

@@ -16,18 +16,18 @@ __global__ __launch_bounds__(NT) void k_row_pass(CartGeom g, const float2 *__res
                                                  double *__restrict__ partial) {
   constexpr bool SUM = MODE == kRowNorm2 || MODE == kRowResidual;
   constexpr bool DUAL = MODE == kRowDualUpdate;
-  __shared__ float2 tile[KIND == kTwo ? kRowTwoElems : RTILE];
-  __shared__ float2 tile2[DUAL && KIND != kTwo ? RTILE : 1];
-  __shared__ float2 twl[api_table_len(KIND)];
-  __shared__ int mrl[KIND == kTwo ? 1 : kRowMaxRows];
+  __shared__ float2 tile[KIND == 0 ? kRowTwoElems : RTILE];
+  __shared__ float2 tile2[DUAL && KIND != 0 ? RTILE : 1];
+  __shared__ float2 twl[row_table_len(KIND)];
+  __shared__ int mrl[KIND == 0 ? 1 : kRowMaxRows];
   __shared__ double red[SUM ? NT : 1];
   double a = 0.0;
-  if constexpr (KIND == kTwo)
+  if constexpr (KIND == 0)
     a = row_two<MODE>(g, blockIdx.x, kcol, z, d, zhat, out, zin, sc, tile, twl);
   else if constexpr (DUAL)
-    row_dual_fused<KIND == kRtWide>(g, blockIdx.x, kcol, z, d, zhat, sc, tile, tile2, twl, mrl);
+    row_dual_fused<KIND == 2>(g, blockIdx.x, kcol, z, d, zhat, sc, tile, tile2, twl, mrl);
   else
-    a = row_mode_fused<MODE, KIND == kRtWide>(g, blockIdx.x, kcol, d, zhat, out, zin, tile, twl,
+    a = row_mode_fused<MODE, KIND == 2>(g, blockIdx.x, kcol, d, zhat, out, zin, tile, twl,
                                               mrl);
   if (SUM) {
     a = block_sum(a, red);
@@ -40,18 +40,17 @@ static void launch_row_kind(const CartGeom &g, int nb, const float2 *kcol, float
                             const float2 *d, float2 *zhat, float2 *out, const float2 *zin,
                             const DevScalars *sc, double *partial, hipStream_t s) {
   const dim3 grid(nb), block(NT);
-  switch (api_kind(g.pw)) {
-    case kTwo: hipLaunchKernelGGL((k_row_pass<MODE, kTwo>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case kRt: hipLaunchKernelGGL((k_row_pass<MODE, kRt>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    default: hipLaunchKernelGGL((k_row_pass<MODE, kRtWide>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
+  switch (row_kind(g)) {
+    case 0: hipLaunchKernelGGL((k_row_pass<MODE, 0>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
+    case 1: hipLaunchKernelGGL((k_row_pass<MODE, 1>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
+    default: hipLaunchKernelGGL((k_row_pass<MODE, 2>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
   }
 }
 
 void launch_row_pass(int mode, const CartGeom &g, const float2 *kcol, float2 *z, const float2 *d,
                      float2 *zhat, float2 *out, const float2 *zin, const DevScalars *sc,
                      double *partial, hipStream_t s) {
-  const int rb = g.pw.ra ? g.RBT : g.RB;
-  const int nb = (int)((g.nrows_c + rb - 1) / rb);
+  const int nb = (int)((g.nrows_c + g.RB - 1) / g.RB);
   if (nb == 0) return;
   switch (mode) {
     case kRowApplyK: launch_row_kind<kRowApplyK>(g, nb, kcol, z, d, zhat, out, zin, sc, partial, s); break;

@@ -84,6 +84,28 @@ static int pick_xb(int H, int W, int emax = EMAX) {
   return xb;
 }
 
+static int log2_ceil(int n) {
+  int l = 0;
+  while ((1 << l) < n) ++l;
+  return l;
+}
+static int col_tile(const CartGeom &g, bool wide) {
+  if (!g.ph.ra) return pick_xb(g.H, g.W, kColTileElems);
+  const int lb = log2_ceil(g.ph.rb), la = log2_ceil(g.ph.ra);
+  int xb = std::min(64, NT >> (wide ? std::max(lb, la - log2_ceil(two_most(g.ph.rb))) : la));
+  while (xb >= 2 * g.W) xb /= 2;
+  return xb;
+}
+void set_col_tiles(CartGeom &g, bool wide) {
+  g.XB = col_tile(g, wide);
+  g.lxb = log2_ceil(g.XB);
+  g.nxb = (g.W + g.XB - 1) / g.XB;
+}
+long wide_col_blocks(const CartGeom &g) {
+  const int xb = col_tile(g, true);
+  return (long)((g.W + xb - 1) / xb) * g.T;
+}
+
 // Radices of a two-stage transform: the pair closest to square (fewest idle
 // lanes), the larger first.
 static void pick_two_stage(FftPlan &p) {
@@ -93,15 +115,6 @@ static void pick_two_stage(FftPlan &p) {
       p.rb = rb;
       return;
     }
-}
-
-static int pick_col_plan(int H, int XBF) {
-  if (H == 256 && XBF == 16) return kColPlan256;
-  if (H == 128 && XBF == 32) return kColPlan128;
-  if (H == 160 && XBF == 16) return kColPlan160;
-  if (H == 192 && XBF == 16) return kColPlan192;
-  if (H == 224 && XBF == 16) return kColPlan224;
-  return kColPlanRt;
 }
 
 void make_fft_plan(int L, FftPlan &p, void **d_tw) {
@@ -144,12 +157,6 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   g = CartGeom{};
   g.W = W; g.H = H; g.C = C; g.T = T;
   g.centered = centered ? 1 : 0;
-  g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / W));
-  g.XBF = pick_xb(H, W, kColTileElems);
-  g.nxbf = (W + g.XBF - 1) / g.XBF;
-  g.cplan = pick_col_plan(H, g.XBF);
-  g.rplan = W == 256 ? kRowPlan256 : (W == 128 ? kRowPlan128 : kRowPlanRt);
-  g.RBF = g.rplan == kRowPlan256 ? 16 : (g.rplan == kRowPlan128 ? 32 : g.RB);
   g.scale = (float)(1.0 / std::sqrt((double)H * W));
   const long HW = (long)H * W;
   std::vector<float> hm;
@@ -207,17 +214,13 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   g.rowmap = (const int *)d_rowmap;
   make_fft_plan(W, g.pw, &d_twx);
   make_fft_plan(H, g.ph, &d_twy);
-  if (g.ph.ra) {
-    g.XB = 1;
-    while (g.XB * 2 * g.ph.ra <= NT && g.XB * 2 <= 64 && g.XB < W) {
-      g.XB *= 2;
-      g.lxb += 1;
-    }
-    g.nxb = (W + g.XB - 1) / g.XB;
-  }
+  set_col_tiles(g, wide_col_blocks(g) >= kColWideBlocks);
   if (g.pw.ra) {
-    while ((1 << g.ljw) < g.pw.ra) g.ljw += 1;
-    g.RBT = NT >> g.ljw;
+    g.ljb = log2_ceil(g.pw.ra);
+    g.lja = std::max(log2_ceil(g.pw.rb), g.ljb - log2_ceil(two_most(g.pw.rb)));
+    g.RB = NT >> g.lja;
+  } else {
+    g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / W));
   }
   g.wide_col = plan_is_wide(g.ph) ? 1 : 0;
   g.wide_row = plan_is_wide(g.pw) ? 1 : 0;

@@ -100,4 +100,11 @@ const char *kernel_name(int id);
 void launch_kernel(int id, int method, int dual_storage, const Task *d_tasks, int n, const TaskGrid &grid,
                    hipStream_t s);
 
+// The Cartesian column and row passes alone (row mode kRowDualUpdate or
+// kRowNorm2), one launch per kind of plan resident.
+void launch_task_col_forward(bool delta, const TaskGrid &grid, const Task *d_tasks, int n,
+                             hipStream_t s);
+void launch_task_col_adjoint(const TaskGrid &grid, const Task *d_tasks, int n, hipStream_t s);
+void launch_task_row(int mode, const TaskGrid &grid, const Task *d_tasks, int n, hipStream_t s);
+
 }  // namespace avionic
