@@ -205,19 +205,24 @@ __device__ __forceinline__ void col_forward_two(const CartGeom &g, int xbi, int 
 // ------------------------------------------------------------ column adjoint
 // Frame t, columns xbi XB ..: transform of the sampled rows along y, times
 // conj(b1_c), summed over the coils in registers.  The coil-map values of a
-// lane's outputs are loaded before its stage-b reads.
-template <class P>
+// lane's outputs are loaded before its stage-b reads.  G groups of NT lanes
+// each take a contiguous share of the coils on a tile of their own (`elems`
+// apart) and add their sums in group order at the end.
+template <class P, int G>
 __device__ __forceinline__ void col_adjoint_two(const CartGeom &g, int xbi, int t,
                                                 const float2 *zhat, const float2 *b1, float2 *out,
-                                                float2 *tile, float2 *twl, int *rml) {
-  const int tid = threadIdx.x;
+                                                float2 *tile, int elems, float2 *twl, int *rml) {
+  const int tid = G > 1 ? threadIdx.x & (NT - 1) : threadIdx.x;
+  const int grp = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  float2 *const tiles = tile;
+  tile += grp * elems;
   const P plan(g);
   const int Ra = plan.ra, Rb = plan.rb, lxb = plan.lxb, H = Ra * Rb;
   int W = g.W;
   const long HW = (long)H * W;
   const bool cen = g.centered != 0;
-  const float2 *tw = stage_twiddles(g.ph, twl, tid, NT);
-  for (int i = tid; i < H; i += NT) rml[i] = g.rowmap[(long)t * H + i];
+  const float2 *tw = stage_twiddles(g.ph, twl, threadIdx.x, NT * G);
+  for (int i = threadIdx.x; i < H; i += NT * G) rml[i] = g.rowmap[(long)t * H + i];
   const int b = tid & ((1 << lxb) - 1);
   int j = tid >> lxb;
   const int jq = NT >> lxb;
@@ -238,14 +243,17 @@ __device__ __forceinline__ void col_adjoint_two(const CartGeom &g, int xbi, int 
   float2 acc[kMaxRadix];
 #pragma unroll
   for (int r = 0; r < kMaxRadix; ++r) acc[r] = czero();
-  for (int c = 0; c < g.C; ++c) {
+  const int share = (g.C + G - 1) / G;
+  for (int ci = 0; ci < share; ++ci) {
+    const int c = grp * share + ci;
+    const bool live = G == 1 || c < g.C;  // uniform over a wave
     j = opaque(j);
     W = opaque_s(W);
     const float2 *bc = b1 + c * HW;
     const BoundedLoad zh(zhat + ((long)g.C * r0 + (long)c * S) * W, 8u * (unsigned)(S * W));
     plan.stage_a([&](auto rc) {
       constexpr int R = decltype(rc)::value;
-      if (j < Rb) {
+      if (live && j < Rb) {
         float2 v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = zh(ko[r]);
@@ -263,7 +271,7 @@ __device__ __forceinline__ void col_adjoint_two(const CartGeom &g, int xbi, int 
 #pragma unroll
       for (int q = 0; q < P::most(R); ++q) {
         const int jj = j + q * jq;
-        if (jj < Ra) {
+        if (live && jj < Ra) {
           float2 m[R], v[R];
           const ImageCol<R> ic(jj, Ra, H, W, xc, cen);
 #pragma unroll
@@ -281,6 +289,40 @@ __device__ __forceinline__ void col_adjoint_two(const CartGeom &g, int xbi, int 
       }
     });
     __syncthreads();
+  }
+  if constexpr (G > 1) {
+    // every group's sums to its tile, then each group finishes its part
+    plan.stage_b([&](auto rc) {
+      constexpr int R = decltype(rc)::value;
+#pragma unroll
+      for (int q = 0; q < P::most(R); ++q) {
+        const int jj = j + q * jq;
+        if (jj < Ra)
+#pragma unroll
+          for (int r = 0; r < R; ++r) tile[((jj + r * Ra) << lxb) + b] = acc[q * R + r];
+      }
+    });
+    __syncthreads();
+    plan.stage_b([&](auto rc) {
+      constexpr int R = decltype(rc)::value;
+#pragma unroll
+      for (int q = 0; q < P::most(R); ++q) {
+        const int jj = j + q * jq;
+        if (jj < Ra && x < W) {
+          const ImageCol<R> ic(jj, Ra, H, W, xc, cen);
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            if (r % G != grp) continue;
+            const float2 *p = tiles + ((jj + r * Ra) << lxb) + b;
+            float2 a = p[0];
+#pragma unroll
+            for (int k = 1; k < G; ++k) a = cadd(a, p[k * elems]);
+            ic.store(out + t * HW, r, cscale(a, g.scale));
+          }
+        }
+      }
+    });
+    return;
   }
   plan.stage_b([&](auto rc) {
     constexpr int R = decltype(rc)::value;

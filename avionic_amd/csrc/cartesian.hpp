@@ -13,6 +13,7 @@
 // the adjoint's row transform are fused into the forward row pass.
 #pragma once
 
+#include <algorithm>
 #include <vector>
 
 #include "common.hpp"
@@ -93,6 +94,15 @@ void set_col_tiles(CartGeom &g, bool wide);
 // are taken: two blocks per CU.
 long wide_col_blocks(const CartGeom &g);
 constexpr long kColWideBlocks = 512;
+
+// Coil groups of a forward column pass of `tiles` blocks (each block takes one
+// group's coils; the results do not depend on it): enough for four blocks per
+// CU.  Measured on MI355X (K, 1 group / this many): 180x240x20x12 (300 tiles)
+// 58 -> 47 us, 192x192x20x10 45 -> 35, 160x160x12x8 28.5 -> 20, 128x128x12x8
+// 25 -> 15; more groups than that re-read the image for nothing.
+inline int col_coil_groups(long tiles, int C) {
+  return (int)std::min<long>(C, std::max<long>(1, 1024 / std::max<long>(1, tiles)));
+}
 
 void make_fft_plan(int L, FftPlan &p, void **d_tw);
 

@@ -272,6 +272,9 @@ struct avionic_engine {
     }
     g.grid.col = bc;
     g.grid.row = br;
+    int coils = 1;
+    for (const Slot *s : g.slots) coils = std::max(coils, s->C);
+    g.grid.col_groups = col_coil_groups(bc, coils);
     if (!tasks.empty()) {
       g.table.ensure(sizeof(Task) * tasks.size());
       AV_HIP(hipMemcpyAsync(g.table.p, tasks.data(), sizeof(Task) * tasks.size(),

@@ -3,7 +3,8 @@
 // One kernel per kind of plan (col_kind, row_kind); a launch covers its kind's
 // span of blocks and is made only when such a task is resident.  DELTA =
 // false: K of the extragradient image (dual update); DELTA = true: K of
-// ext - x (step rule, adapting tasks only).
+// ext - x (step rule, adapting tasks only).  The forward column pass of a
+// small launch set splits each task's coils into `groups` blocks per tile.
 #include "cart_two.hpp"
 #include "tasks_device.hpp"
 
@@ -11,7 +12,7 @@ namespace avionic {
 
 template <bool DELTA, int KIND>
 __global__ __launch_bounds__(NTC) void kt_col_forward(const Task *__restrict__ tasks, int n,
-                                                      int blk0) {
+                                                      int blk0, int groups) {
   __shared__ float2 tile[KIND & 1 ? kColTwoElems : kColTileElems];
   __shared__ float2 twl[col_table_len(KIND)];
   __shared__ int rml[col_table_len(KIND)];
@@ -21,13 +22,15 @@ __global__ __launch_bounds__(NTC) void kt_col_forward(const Task *__restrict__ t
   if (!task_active(T.sc)) return;
   if (DELTA && !task_adapt(T.sc)) return;
   const int lb = blk - T.b_col, xbi = lb % T.cg.nxb, t = lb / T.cg.nxb;
+  const int cpg = (T.cg.C + groups - 1) / groups, c0 = (int)blockIdx.y * cpg;
+  const int c1 = min(T.cg.C, c0 + cpg);
   const float2 *usub = DELTA ? T.x : nullptr;
   if constexpr (KIND == 1)
-    col_forward_two<DELTA, TwoRt>(T.cg, xbi, t, 0, T.cg.C, T.ext, usub, T.b1, T.kcol, tile, twl, rml);
+    col_forward_two<DELTA, TwoRt>(T.cg, xbi, t, c0, c1, T.ext, usub, T.b1, T.kcol, tile, twl, rml);
   else if constexpr (KIND == 3)
-    col_forward_two<DELTA, Two256>(T.cg, xbi, t, 0, T.cg.C, T.ext, usub, T.b1, T.kcol, tile, twl, rml);
+    col_forward_two<DELTA, Two256>(T.cg, xbi, t, c0, c1, T.ext, usub, T.b1, T.kcol, tile, twl, rml);
   else
-    col_forward_fused<DELTA, KIND == 2>(T.cg, xbi, t, 0, T.cg.C, T.ext, usub, T.b1, T.kcol, tile,
+    col_forward_fused<DELTA, KIND == 2>(T.cg, xbi, t, c0, c1, T.ext, usub, T.b1, T.kcol, tile,
                                         twl, rml);
 }
 
@@ -75,9 +78,9 @@ void kt_col_adjoint(const Task *__restrict__ tasks, int n, int blk0) {
   if (!task_active(T.sc)) return;
   const int lb = blk - T.b_col, xbi = lb % T.cg.nxb, t = lb / T.cg.nxb;
   if constexpr (KIND == 1)
-    col_adjoint_two<TwoRt>(T.cg, xbi, t, T.zhat, T.b1, T.khz, tile, twl, rml);
+    col_adjoint_two<TwoRt, 1>(T.cg, xbi, t, T.zhat, T.b1, T.khz, tile, 0, twl, rml);
   else if constexpr (KIND == 3)
-    col_adjoint_two<Two256>(T.cg, xbi, t, T.zhat, T.b1, T.khz, tile, twl, rml);
+    col_adjoint_two<Two256, 1>(T.cg, xbi, t, T.zhat, T.b1, T.khz, tile, 0, twl, rml);
   else
     col_adjoint_fused<KIND == 2>(T.cg, xbi, t, T.zhat, T.b1, T.khz, tile, twl, rml);
 }
@@ -87,8 +90,8 @@ static void col_fwd(const TaskGrid &gr, const Task *d_tasks, int n, hipStream_t 
   if constexpr (K < kColKinds) {
     const int nb = gr.col_hi[K] - gr.col_lo[K];
     if (nb > 0)
-      hipLaunchKernelGGL((kt_col_forward<DELTA, K>), dim3(nb), dim3(NTC), 0, s, d_tasks, n,
-                         gr.col_lo[K]);
+      hipLaunchKernelGGL((kt_col_forward<DELTA, K>), dim3(nb, gr.col_groups), dim3(NTC), 0, s, d_tasks, n,
+                         gr.col_lo[K], gr.col_groups);
     col_fwd<DELTA, K + 1>(gr, d_tasks, n, s);
   }
 }

@@ -53,6 +53,7 @@ struct Task {
 // tasks: device array; the host mirror gives the grid sizes.
 struct TaskGrid {
   int vox = 0, col = 0, row = 0;
+  int col_groups = 1;  // coil groups of the forward column pass (col_coil_groups)
   // Dual / primal blocks of the one-voxel-per-lane and the pair tasks.
   int dp1 = 0, dp2 = 0;
   // Launch variant (both give the same bits): lanes 2 runs pairs of voxels

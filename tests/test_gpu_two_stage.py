@@ -32,3 +32,18 @@ def test_operator_pair_every_radix(gpu, W, H, centered):
                 assert not np.any(got)
             else:
                 assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 2e-6
+
+
+@pytest.mark.parametrize("W,H,T,C", [(40, 36, 2, 1), (40, 36, 2, 2), (40, 36, 2, 3), (40, 36, 2, 4),
+                                     (48, 256, 2, 7), (50, 225, 3, 9), (16, 64, 90, 4), (72, 64, 170, 3)])
+def test_operator_pair_coil_groups(gpu, W, H, T, C):
+    """Coil counts that the blocks' coil groups do not divide, a group without
+    a coil, and grids on both sides of the sizes where the groups start."""
+    print(f"[gpu coil groups] W={W} H={H} T={T} C={C}", flush=True)
+    rng = np.random.default_rng(C)
+    c = lambda *s: (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64).astype(np.complex128)
+    x, b1, z = c(T, H, W), c(C, H, W), c(T, C, H, W)
+    mask = np.repeat((rng.random((T, H, 1)) < 0.5).astype(np.float64), W, axis=2)
+    for got, ref in ((gpu.cart_K(x, b1, mask, False), O.cart_K(x, b1, mask, False)),
+                     (gpu.cart_KH(z, b1, mask, False), O.cart_KH(z, b1, mask, False))):
+        assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 2e-6
