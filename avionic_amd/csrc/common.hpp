@@ -297,14 +297,30 @@ struct FftPlan {
   int radix[kMaxStages];
   int ns[kMaxStages];
   int ra, rb;        // L = ra rb with 16 >= ra >= rb (0: no such pair)
+  // The float transforms' stages: radices up to 16, composites among them
+  // (plan_radix), the product L with the least work per element; at least two
+  // stages (the rest radix 1).
+  int nx;
+  int rx[kMaxStages];
   const float2 *tw;  // tw[m] = exp(-2 pi i m / L), m < L (device)
 };
+// Radices of rx; 11 and 13 run in the wide kernels only.  14 and 15 are left
+// out: 256 lanes hold two of their butterflies at a 4096-element tile, 30
+// values for the 16 of the others.
+__host__ __device__ constexpr bool plan_radix(int r, bool wide) {
+  return r != 14 && r != 15 && (wide || (r != 11 && r != 13));
+}
 __host__ __device__ inline bool plan_is_wide(const FftPlan &p) {
   if (p.L > kMaxFftLenNarrow) return true;
   for (int s = 0; s < p.nst; ++s)
     if (p.radix[s] == 11 || p.radix[s] == 13) return true;
   return false;
 }
+
+// How fft_io runs a plan (its WIDE argument): rx on narrow or wide kernels, or
+// the two stages ra, rb with one butterfly per lane (transforms per call times
+// ra at most the lanes).
+enum PlanKind { kPlanNarrow = 0, kPlanWide = 1, kPlanTwo = 2 };
 
 // ----------------------------------------------------- reductions / state
 constexpr int kRedThreads = 256;

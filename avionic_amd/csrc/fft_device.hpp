@@ -237,80 +237,24 @@ __device__ __forceinline__ void with_radix(int R, F &&f) {
   }
 }
 
-// One Stockham stage.  Must be called by all NT threads of the block.
-// BFAST: consecutive lanes take consecutive transforms (b) instead of
-// consecutive butterflies (j); pick the one whose LDS stride is 1.
-template <int R, int NT, int EMAX, bool BFAST>
-__device__ inline void fft_stage(float2 *buf, int L, int B, int bstride, int istride, int Ns,
-                                 float sign, const float2 *__restrict__ tw, int tid) {
-  constexpr int MAXB = (EMAX / R + NT - 1) / NT;
-  // Opaque copy of the lane id: keeps the compiler from hoisting each radix's
-  // per-lane index arithmetic out of the stage loop (which would keep every
-  // radix's indices live at once and multiply the register footprint).
-  asm volatile("" : "+v"(tid));
-  const int nbf = L / R;
-  const int total = nbf * B;
-  const int twstep = L / (Ns * R);
-  const int rstride = nbf * istride;
-  float2 v[MAXB][R];
-#pragma unroll
-  for (int c = 0; c < MAXB; ++c) {
-    const int idx = tid + c * NT;
-    if (idx < total) {
-      int b, j;
-      if (BFAST) { b = idx % B; j = idx / B; } else { j = idx % nbf; b = idx / nbf; }
-      const int k = j % Ns;
-      const int base = b * bstride + j * istride;
-      v[c][0] = buf[base];
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        float2 w = tw[r * k * twstep];
-        w.y = -sign * w.y;  // tw holds exp(-i theta); want exp(sign i theta)
-        v[c][r] = cmul(buf[base + r * rstride], w);
-      }
-      Dft<R>::run(v[c], sign);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int c = 0; c < MAXB; ++c) {
-    const int idx = tid + c * NT;
-    if (idx < total) {
-      int b, j;
-      if (BFAST) { b = idx % B; j = idx / B; } else { j = idx % nbf; b = idx / nbf; }
-      const int k = j % Ns;
-      const int base = b * bstride + ((j / Ns) * Ns * R + k) * istride;
-      const int ostride = Ns * istride;
-#pragma unroll
-      for (int r = 0; r < R; ++r) buf[base + r * ostride] = v[c][r];
-    }
-  }
-  __syncthreads();
+// a / n for 0 <= a < 2^13, 1 <= n: folded where n is a constant, else one
+// reciprocal (its error is far below the 0.5 / n that separates a + 0.5 from
+// the next multiple of n).
+__device__ __forceinline__ int small_div(int a, int n) {
+  if (__builtin_constant_p(n)) return a / n;
+  return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)n));
 }
-
-// Full transform of B batched length-L sequences in LDS (unnormalised).
-// Radices 11 and 13 are compiled in only with WIDE (see plan_is_wide).
-template <int NT, int EMAX, bool BFAST, bool WIDE = true>
-__device__ inline void fft_lds(float2 *buf, const FftPlan &p, int B, int bstride, int istride,
-                               float sign, int tid) {
-  for (int s = 0; s < p.nst; ++s) {
-    const int R = p.radix[s], Ns = p.ns[s];
-    switch (R) {
-      case 16: fft_stage<16, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 8: fft_stage<8, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 4: fft_stage<4, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 2: fft_stage<2, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 3: fft_stage<3, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 5: fft_stage<5, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 7: fft_stage<7, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid); break;
-      case 11:
-        if constexpr (WIDE) fft_stage<11, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid);
-        break;
-      case 13:
-        if constexpr (WIDE) fft_stage<13, NT, EMAX, BFAST>(buf, p.L, B, bstride, istride, Ns, sign, p.tw, tid);
-        break;
-      default: break;
-    }
+// Butterfly j of transform b from a lane's index: BFAST (B a power of two)
+// takes consecutive transforms on consecutive lanes, else consecutive
+// butterflies.
+template <bool BFAST>
+__device__ __forceinline__ void butterfly_of(int idx, int nbf, int B, int &b, int &j) {
+  if (BFAST) {
+    b = idx & (B - 1);
+    j = idx >> (31 - __clz(B));
+  } else {
+    b = small_div(idx, nbf);
+    j = idx - b * nbf;
   }
 }
 
@@ -343,8 +287,8 @@ __device__ __forceinline__ void fft_stage_io(float2 *buf, int L, int B, int bstr
     const int idx = tid + c * NT;
     if (idx < total) {
       int b, j;
-      if (BFAST) { b = idx % B; j = idx / B; } else { j = idx % nbf; b = idx / nbf; }
-      const int k = j % Ns;
+      butterfly_of<BFAST>(idx, nbf, B, b, j);
+      const int m = Ns > 1 ? small_div(j, Ns) : j, k = j - m * Ns;
       if (FROMG) {
 #pragma unroll
         for (int r = 0; r < R; ++r) v[c][r] = ld(b, j + r * nbf, c * R + r);
@@ -370,9 +314,9 @@ __device__ __forceinline__ void fft_stage_io(float2 *buf, int L, int B, int bstr
     const int idx = tid + c * NT;
     if (idx < total) {
       int b, j;
-      if (BFAST) { b = idx % B; j = idx / B; } else { j = idx % nbf; b = idx / nbf; }
-      const int k = j % Ns;
-      const int o = (j / Ns) * Ns * R + k;
+      butterfly_of<BFAST>(idx, nbf, B, b, j);
+      const int m = Ns > 1 ? small_div(j, Ns) : j, k = j - m * Ns;
+      const int o = m * Ns * R + k;
       if (TOG) {
 #pragma unroll
         for (int r = 0; r < R; ++r) st(b, o + r * Ns, v[c][r], c * R + r);
@@ -387,26 +331,64 @@ __device__ __forceinline__ void fft_stage_io(float2 *buf, int L, int B, int bstr
   if (!TOG) __syncthreads();
 }
 
-template <int NT, int EMAX, bool BFAST, bool FROMG, bool TOG, bool WIDE, class LD, class ST>
-__device__ inline void fft_stage_io_dispatch(int R, float2 *buf, int L, int B, int bstride,
+template <int NT, int EMAX, bool BFAST, bool FROMG, bool TOG, int WIDE, class LD, class ST>
+__device__ __forceinline__ void fft_stage_io_dispatch(int R, float2 *buf, int L, int B, int bstride,
                                              int istride, int Ns, float sign, const float2 *tw,
                                              int tid, LD &ld, ST &st) {
+  // (written out: through with_radix's closure the functors' per-lane arrays
+  // stay in scratch memory)
+#define AV_CASE(r)                                                                            \
+  if constexpr (plan_radix(r, WIDE == kPlanWide))                                             \
+  fft_stage_io<r, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, \
+                                               ld, st)
   switch (R) {
-    case 16: fft_stage_io<16, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 8: fft_stage_io<8, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 4: fft_stage_io<4, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 2: fft_stage_io<2, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 3: fft_stage_io<3, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 5: fft_stage_io<5, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 7: fft_stage_io<7, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st); break;
-    case 11:
-      if constexpr (WIDE) fft_stage_io<11, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st);
-      break;
-    case 13:
-      if constexpr (WIDE) fft_stage_io<13, NT, EMAX, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, ld, st);
-      break;
-    default: break;
+    case 16: AV_CASE(16); break;
+    case 15: AV_CASE(15); break;
+    case 14: AV_CASE(14); break;
+    case 13: AV_CASE(13); break;
+    case 12: AV_CASE(12); break;
+    case 11: AV_CASE(11); break;
+    case 10: AV_CASE(10); break;
+    case 9: AV_CASE(9); break;
+    case 8: AV_CASE(8); break;
+    case 7: AV_CASE(7); break;
+    case 6: AV_CASE(6); break;
+    case 5: AV_CASE(5); break;
+    case 4: AV_CASE(4); break;
+    case 3: AV_CASE(3); break;
+    case 2: AV_CASE(2); break;
+    default: AV_CASE(1); break;
   }
+#undef AV_CASE
+}
+// Two-stage transforms (plan_kind kPlanTwo) whose lanes hold at most one butterfly of each stage
+// (B ra <= NT): any radix up to 16 with one butterfly's registers.
+template <int NT, bool BFAST, bool FROMG, bool TOG, class LD, class ST>
+__device__ __forceinline__ void fft_stage_one(int R, float2 *buf, int L, int B, int bstride, int istride,
+                                     int Ns, float sign, const float2 *tw, int tid, LD &ld,
+                                     ST &st) {
+#define AV_CASE(r)                                                                               \
+  fft_stage_io<r, NT, r * NT, BFAST, FROMG, TOG>(buf, L, B, bstride, istride, Ns, sign, tw, tid, \
+                                                 ld, st)
+  switch (R) {
+    case 16: AV_CASE(16); break;
+    case 15: AV_CASE(15); break;
+    case 14: AV_CASE(14); break;
+    case 13: AV_CASE(13); break;
+    case 12: AV_CASE(12); break;
+    case 11: AV_CASE(11); break;
+    case 10: AV_CASE(10); break;
+    case 9: AV_CASE(9); break;
+    case 8: AV_CASE(8); break;
+    case 7: AV_CASE(7); break;
+    case 6: AV_CASE(6); break;
+    case 5: AV_CASE(5); break;
+    case 4: AV_CASE(4); break;
+    case 3: AV_CASE(3); break;
+    case 2: AV_CASE(2); break;
+    default: AV_CASE(1); break;
+  }
+#undef AV_CASE
 }
 
 struct NoLoad {
@@ -416,13 +398,13 @@ struct NoStore {
   __device__ void operator()(int, int, float2, int) {}
 };
 
-// Outputs per lane of one stage: max over radices of ceil(EMAX/R/NT) * R
-// (radices 11 and 13 only in wide kernels).
-constexpr int max_slots(int emax, int nt, bool wide) {
+// Outputs per lane of one stage: max over a plan's radices of
+// ceil(EMAX/R/NT) * R.
+constexpr int max_slots(int emax, int nt, int kind) {
+  if (kind == kPlanTwo) return kMaxRadix;
   int m = 0;
-  const int rs[] = {16, 8, 4, 2, 3, 5, 7, 11, 13};
-  for (int r : rs) {
-    if (!wide && r > 8 && r != 16) continue;
+  for (int r = 2; r <= kMaxRadix; ++r) {
+    if (!plan_radix(r, kind == kPlanWide)) continue;
     const int v = ((emax / r + nt - 1) / nt) * r;
     m = v > m ? v : m;
   }
@@ -434,37 +416,34 @@ constexpr int max_slots(int emax, int nt, bool wide) {
 // before re-using a tile.  With TOG the LDS tile is free once this returns
 // (the last stage read it before the function's final store loop; lanes may
 // still be reading it, so callers sync before writing the tile again).
-template <int NT, int EMAX, bool BFAST, bool FROMG, bool TOG, bool WIDE, class LD, class ST>
-__device__ inline void fft_io(float2 *buf, const FftPlan &p, int B, int bstride, int istride,
+template <int NT, int EMAX, bool BFAST, bool FROMG, bool TOG, int WIDE, class LD, class ST>
+__device__ __forceinline__ void fft_io(float2 *buf, const FftPlan &p, int B, int bstride, int istride,
                               float sign, int tid, const float2 *tw, LD &ld, ST &st) {
-  const int n = p.nst;
-  if (n == 0) {  // length 1: identity
-    for (int b = tid; b < B; b += NT) {
-      const float2 v = FROMG ? ld(b, 0, 0) : buf[b * bstride];
-      if (TOG) st(b, 0, v, 0); else buf[b * bstride] = v;
-    }
-    if (!TOG) __syncthreads();
-    return;
-  }
-  if (n == 1) {
-    fft_stage_io_dispatch<NT, EMAX, BFAST, FROMG, TOG, WIDE>(p.radix[0], buf, p.L, B, bstride, istride,
-                                                       p.ns[0], sign, tw, tid, ld, st);
-    return;
-  }
   NoStore ns;
   NoLoad nl;
-  fft_stage_io_dispatch<NT, EMAX, BFAST, FROMG, false, WIDE>(p.radix[0], buf, p.L, B, bstride, istride,
-                                                       p.ns[0], sign, tw, tid, ld, ns);
-  for (int s = 1; s < n - 1; ++s)
-    fft_stage_io_dispatch<NT, EMAX, BFAST, false, false, WIDE>(p.radix[s], buf, p.L, B, bstride, istride,
-                                                         p.ns[s], sign, tw, tid, nl, ns);
-  fft_stage_io_dispatch<NT, EMAX, BFAST, false, TOG, WIDE>(p.radix[n - 1], buf, p.L, B, bstride, istride,
-                                                     p.ns[n - 1], sign, tw, tid, nl, st);
+  if constexpr (WIDE == kPlanTwo) {
+    fft_stage_one<NT, BFAST, FROMG, false>(p.ra, buf, p.L, B, bstride, istride, 1, sign, tw, tid,
+                                           ld, ns);
+    fft_stage_one<NT, BFAST, false, TOG>(p.rb, buf, p.L, B, bstride, istride, p.ra, sign, tw, tid,
+                                         nl, st);
+  } else {
+  const int n = p.nx;  // at least 2
+  fft_stage_io_dispatch<NT, EMAX, BFAST, FROMG, false, WIDE>(p.rx[0], buf, p.L, B, bstride, istride,
+                                                       1, sign, tw, tid, ld, ns);
+  int Ns = p.rx[0];
+  for (int s = 1; s < n - 1; ++s) {
+    fft_stage_io_dispatch<NT, EMAX, BFAST, false, false, WIDE>(p.rx[s], buf, p.L, B, bstride, istride,
+                                                         Ns, sign, tw, tid, nl, ns);
+    Ns *= p.rx[s];
+  }
+  fft_stage_io_dispatch<NT, EMAX, BFAST, false, TOG, WIDE>(p.rx[n - 1], buf, p.L, B, bstride, istride,
+                                                     Ns, sign, tw, tid, nl, st);
+  }
 }
 
 // A plan known at compile time: length L = R0 R1 R2, stages in that order
 // (R2 = 1: two stages).  fft_io_ct runs the stages fft_io runs on
-// make_fft_plan's plan of the same radices (same butterflies, twiddle indices
+// a plan of the same radices (same butterflies, twiddle indices
 // and Stockham positions), with the length, the stage strides and, for
 // BFAST, the transform count folded into constants: the per-element index
 // divisions and remainders of the runtime plan become multiplies and shifts.

@@ -23,53 +23,68 @@ __global__ void k_compact_gather(CartGeom g, const float2 *__restrict__ dense,
 
 // Standalone batched 2D FFT (used by avionic_fft2, the AGILE FFT
 // replacement): rows out of place (the centred y shift permutes rows between
-// blocks), then columns in place.
+// blocks), then columns in place.  Each stage chain reads its first stage from
+// global memory and writes its last stage there.
+struct FftRowLoad {
+  const float2 *base;  // image
+  int H, W, y0, centered;
+  __device__ float2 operator()(int b, int i, int) const {
+    const int y = centered ? wrap_half(y0 + b, H) : y0 + b;
+    return gld(base, (unsigned)(y * W + (centered ? wrap_half(i, W) : i)));
+  }
+};
+struct FftRowStore {
+  float2 *base;  // image row y0
+  int W, centered;
+  __device__ void operator()(int b, int i, float2 v, int) const {
+    gst(base, (unsigned)(b * W + (centered ? wrap_half(i, W) : i)), v);
+  }
+};
+template <int KIND>
 __global__ __launch_bounds__(NT) void k_fft_rows_oop(const float2 *in, float2 *outp, FftPlan pw,
                                                      int H, int W, int RB, int sign,
                                                      int centered) {
   __shared__ float2 tile[EMAX];
+  __shared__ float2 twl[KIND == kPlanWide ? kMaxFftLen : kMaxFftLenNarrow];
   const int tid = threadIdx.x;
-  const long img = blockIdx.y;
+  const long img = (long)blockIdx.y * H * W;
   const int y0 = blockIdx.x * RB;
-  const int nr = min(RB, H - y0);
-  const float2 *base = in + img * (long)H * W;
-  float2 *ob = outp + img * (long)H * W;
-  for (int e = tid; e < nr * W; e += NT) {
-    const int r = e / W, x = e % W;
-    const int y = y0 + r;
-    const int sy = centered ? (y + H / 2) % H : y;
-    const int sx = centered ? (x + W / 2) % W : x;
-    tile[e] = base[(long)sy * W + sx];
-  }
+  const float2 *tw = stage_twiddles(pw, twl, tid, NT);
   __syncthreads();
-  fft_lds<NT, EMAX, false>(tile, pw, nr, W, 1, (float)sign, tid);
-  const int wc = (W + 1) / 2;
-  for (int e = tid; e < nr * W; e += NT) {
-    const int r = e / W, kx = e % W;
-    const int src = centered ? (kx + wc) % W : kx;
-    ob[(long)(y0 + r) * W + kx] = tile[r * W + src];
-  }
+  FftRowLoad ld{in + img, H, W, y0, centered};
+  FftRowStore st{outp + img + (long)y0 * W, W, centered};
+  fft_io<NT, EMAX, false, true, true, KIND>(tile, pw, min(RB, H - y0), W, 1, (float)sign, tid, tw,
+                                            ld, st);
 }
 
+struct FftColLoad {
+  const float2 *base;  // image column xb0
+  int W, nx;
+  __device__ float2 operator()(int b, int i, int) const {
+    return gld(base, (unsigned)(i * W + min(b, nx - 1)));  // columns past the last: dropped
+  }
+};
+struct FftColStore {
+  float2 *base;
+  int H, W, nx, centered;
+  float scale;
+  __device__ void operator()(int b, int i, float2 v, int) const {
+    if (b < nx) gst(base, (unsigned)((centered ? wrap_half(i, H) : i) * W + b), cscale(v, scale));
+  }
+};
+template <int KIND>
 __global__ __launch_bounds__(NT) void k_fft_cols(float2 *data, FftPlan ph, int H, int W, int XB,
                                                  int sign, int centered, float scale) {
   __shared__ float2 tile[EMAX];
+  __shared__ float2 twl[KIND == kPlanWide ? kMaxFftLen : kMaxFftLenNarrow];
   const int tid = threadIdx.x;
-  const long img = blockIdx.y;
   const int xb0 = blockIdx.x * XB;
-  float2 *base = data + img * (long)H * W;
-  for (int e = tid; e < H * XB; e += NT) {
-    const int y = e / XB, x = xb0 + e % XB;
-    tile[e] = (x < W) ? base[(long)y * W + x] : czero();
-  }
+  float2 *base = data + (long)blockIdx.y * H * W + xb0;
+  const float2 *tw = stage_twiddles(ph, twl, tid, NT);
   __syncthreads();
-  fft_lds<NT, EMAX, true>(tile, ph, XB, 1, XB, (float)sign, tid);
-  const int hc = (H + 1) / 2;
-  for (int e = tid; e < H * XB; e += NT) {
-    const int y = e / XB, x = xb0 + e % XB;
-    const int src = centered ? (y + hc) % H : y;
-    if (x < W) base[(long)y * W + x] = cscale(tile[src * XB + e % XB], scale);
-  }
+  FftColLoad ld{base, W, min(XB, W - xb0)};
+  FftColStore st{base, H, W, min(XB, W - xb0), centered, scale};
+  fft_io<NT, EMAX, true, true, true, KIND>(tile, ph, XB, 1, XB, (float)sign, tid, tw, ld, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -117,6 +132,29 @@ static void pick_two_stage(FftPlan &p) {
     }
 }
 
+// Stages of the float transforms: over the factorisations of L into plan
+// radices (largest first), the one with the least work per element: a
+// radix's own operations, the twiddles after the first stage, and about 8
+// operations for the stage's LDS round trip and indices.
+static void pick_stages(int m, int most, double cost, int n, int *r, double &best, FftPlan &p) {
+  static const double ops[kMaxRadix + 1] = {0, 0, 2, 5.3, 4, 8, 7.3, 11.5, 6.5, 10, 10, 17, 9.3,
+                                            20, 0, 0, 10.5};
+  if (m == 1) {
+    if (cost < best) {
+      best = cost;
+      p.nx = n;
+      std::copy(r, r + n, p.rx);
+    }
+    return;
+  }
+  if (n == kMaxStages) return;
+  for (int q = std::min(most, m); q >= 2; --q)
+    if (m % q == 0 && plan_radix(q, true)) {
+      r[n] = q;
+      pick_stages(m / q, q, cost + ops[q] + 8 + (n ? 4 : 0), n + 1, r, best, p);
+    }
+}
+
 void make_fft_plan(int L, FftPlan &p, void **d_tw) {
   AV_CHECK(L >= 1 && L <= kMaxFftLen, "FFT length out of range (1..1024)");
   p = FftPlan{};
@@ -135,6 +173,10 @@ void make_fft_plan(int L, FftPlan &p, void **d_tw) {
   }
   AV_CHECK(m == 1, "FFT length must factor into 2, 3, 5, 7, 11 and 13");
   pick_two_stage(p);
+  int r[kMaxStages];
+  double best = 1e30;
+  pick_stages(L, kMaxRadix, 0.0, 0, r, best, p);
+  while (p.nx < 2) p.rx[p.nx++] = 1;
   std::vector<float2> tw(L);
   for (int k = 0; k < L; ++k) {
     const double a = -2.0 * M_PI * (double)k / (double)L;
@@ -240,18 +282,38 @@ void launch_compact_gather(const CartGeom &g, const float2 *dense, float2 *compa
   AV_LAUNCH_CHECK();
 }
 
+// fft_io's kind for B transforms of a plan per block.
+static int plan_kind(const FftPlan &p, int B) {
+  if (p.ra && B * p.ra <= NT) return kPlanTwo;
+  return plan_is_wide(p) ? kPlanWide : kPlanNarrow;
+}
+
+static void launch_cols(float2 *data, const FftPlan &p, int L, int plane, int batch, int sign,
+                        int centered, float scale, hipStream_t s) {
+  int XB = pick_xb(L, plane);
+  while (p.ra && XB > 1 && XB * p.ra > NT) XB /= 2;
+  const dim3 grid((plane + XB - 1) / XB, batch), block(NT);
+  switch (plan_kind(p, XB)) {
+    case kPlanTwo: hipLaunchKernelGGL(k_fft_cols<kPlanTwo>, grid, block, 0, s, data, p, L, plane, XB, sign, centered, scale); break;
+    case kPlanWide: hipLaunchKernelGGL(k_fft_cols<kPlanWide>, grid, block, 0, s, data, p, L, plane, XB, sign, centered, scale); break;
+    default: hipLaunchKernelGGL(k_fft_cols<kPlanNarrow>, grid, block, 0, s, data, p, L, plane, XB, sign, centered, scale); break;
+  }
+  AV_LAUNCH_CHECK();
+}
+
 void launch_fft2(float2 *data, const FftPlan &pw, const FftPlan &ph, int H, int W, int batch,
                  int sign, int centered, float scale, hipStream_t s) {
-  const int RB = EMAX / W;
+  const int RB = pw.ra ? std::min(EMAX / W, NT / pw.ra) : EMAX / W;
   float2 *tmp = nullptr;
   AV_HIP(hipMallocAsync((void **)&tmp, sizeof(float2) * (size_t)H * W * batch, s));
-  hipLaunchKernelGGL(k_fft_rows_oop, dim3((H + RB - 1) / RB, batch), dim3(NT), 0, s, data, tmp, pw, H,
-                     W, RB, sign, centered);
+  const dim3 grid((H + RB - 1) / RB, batch), block(NT);
+  switch (plan_kind(pw, RB)) {
+    case kPlanTwo: hipLaunchKernelGGL(k_fft_rows_oop<kPlanTwo>, grid, block, 0, s, data, tmp, pw, H, W, RB, sign, centered); break;
+    case kPlanWide: hipLaunchKernelGGL(k_fft_rows_oop<kPlanWide>, grid, block, 0, s, data, tmp, pw, H, W, RB, sign, centered); break;
+    default: hipLaunchKernelGGL(k_fft_rows_oop<kPlanNarrow>, grid, block, 0, s, data, tmp, pw, H, W, RB, sign, centered); break;
+  }
   AV_LAUNCH_CHECK();
-  const int XB = pick_xb(H, W);
-  hipLaunchKernelGGL(k_fft_cols, dim3((W + XB - 1) / XB, batch), dim3(NT), 0, s, tmp, ph, H, W, XB,
-                     sign, centered, scale);
-  AV_LAUNCH_CHECK();
+  launch_cols(tmp, ph, H, W, batch, sign, centered, scale, s);
   AV_HIP(hipMemcpyAsync(data, tmp, sizeof(float2) * (size_t)H * W * batch, hipMemcpyDeviceToDevice, s));
   AV_HIP(hipFreeAsync(tmp, s));
 }
@@ -260,10 +322,7 @@ void launch_fft2(float2 *data, const FftPlan &pw, const FftPlan &ph, int H, int 
 // one length-L transform per column of the plane (the depth axis of a volume).
 void launch_fft_axis0(float2 *data, const FftPlan &p, int L, int plane, int batch, int sign,
                       float scale, hipStream_t s) {
-  const int XB = pick_xb(L, plane);
-  hipLaunchKernelGGL(k_fft_cols, dim3((plane + XB - 1) / XB, batch), dim3(NT), 0, s, data, p, L,
-                     plane, XB, sign, 0, scale);
-  AV_LAUNCH_CHECK();
+  launch_cols(data, p, L, plane, batch, sign, 0, scale, s);
 }
 
 }  // namespace avionic

@@ -82,12 +82,12 @@ NcTiles tune_tiles(NcGeom g, float2 *tmp, float2 *part) {
     NcTiles t{kNcFwdCoilGroups, kNcAdjRows};
     if (std::sscanf(force, "%d,%d", &t.cg, &t.rows) == 2) {
       t.cg = std::max(1, std::min(t.cg, g.C));
-      t.rows = std::max(1, std::min(t.rows, std::max(1, 4096 / g.Gx)));
+      t.rows = std::max(1, std::min(t.rows, g.RBf));
       return t;
     }
   }
   const NcTiles def{std::max(1, std::min(g.C, kNcFwdCoilGroups)),
-                    std::max(1, std::min(4096 / g.Gx, kNcAdjRows))};
+                    std::max(1, std::min(g.RBf, kNcAdjRows))};
   const char *tune = std::getenv("AVIONIC_NC_TUNE");
   if (tune && std::strcmp(tune, "0") == 0) return def;
   const std::array<long, 7> key{g.W, g.H, g.C, g.T, g.M, g.Gx, g.Gy};
@@ -117,7 +117,7 @@ NcTiles tune_tiles(NcGeom g, float2 *tmp, float2 *part) {
   g.CG = best.cg;
   bt = 1e30;
   for (int rows : {1, 2, 4, 8}) {
-    if (rows * g.Gx > 4096) break;
+    if (rows > g.RBf) break;
     g.RBa = rows;
     const double t = time_ms([&] {
       launch_nc_adjoint(g, z.as<float2>(), b1.as<float2>(), tmp, img.as<float2>(), s);
@@ -130,9 +130,11 @@ NcTiles tune_tiles(NcGeom g, float2 *tmp, float2 *part) {
   return best;
 }
 
-int pick_cols(int L, int n) {
+// Columns per column-pass block: a two-stage transform holds one butterfly
+// per lane.
+int pick_cols(const FftPlan &p, int n) {
   int xb = 1;
-  while (xb * 2 * L <= 4096 && xb * 2 <= 64 && xb < n) xb *= 2;
+  while (xb * 2 * p.L <= 4096 && xb * 2 <= 64 && xb < n && !(p.ra && xb * 2 * p.ra > 256)) xb *= 2;
   return xb;
 }
 
@@ -297,11 +299,14 @@ class NoncartesianOperator : public Operator {
 
     g_.W = W; g_.H = H; g_.C = C; g_.T = T; g_.M = (int)M;
     g_.Gx = Gx; g_.Gy = Gy;
-    g_.wide = (plan_is_wide(g_.px) || plan_is_wide(g_.py)) ? 1 : 0;
-    g_.XBf = pick_cols(Gy, W);
-    g_.XBa = pick_cols(Gy, Gx);
-    g_.RBf = std::max(1, 4096 / Gx);
-    g_.RBa = std::max(1, std::min(4096 / Gx, kNcAdjRows));
+    g_.XBf = pick_cols(g_.py, W);
+    g_.XBa = pick_cols(g_.py, Gx);
+    // two-stage transforms: one butterfly per lane
+    g_.RBf = g_.px.ra ? std::min(4096 / Gx, 256 / g_.px.ra) : 4096 / Gx;
+    g_.RBa = std::max(1, std::min(g_.RBf, kNcAdjRows));
+    g_.wide = (plan_is_wide(g_.px) || plan_is_wide(g_.py)) ? kPlanWide : kPlanNarrow;
+    if (g_.px.ra && g_.py.ra && std::max(g_.XBf, g_.XBa) * g_.py.ra <= 256 && g_.RBf * g_.px.ra <= 256)
+      g_.wide = kPlanTwo;  // one butterfly per lane in every pass (RBa at most RBf)
     g_.CG = std::max(1, std::min(C, kNcFwdCoilGroups));
     g_.scale = (float)sc;
     g_.dxi = dxi_.as<float>();
