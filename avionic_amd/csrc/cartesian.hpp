@@ -119,6 +119,8 @@ void launch_col_adjoint(const CartGeom &g, const float2 *zhat, const float2 *b1,
                         hipStream_t s);
 // Gather dense [t][c][H][W] k-space rows into compact storage (times mask).
 void launch_compact_gather(const CartGeom &g, const float2 *dense, float2 *compact, hipStream_t s);
+// fft_io's kind (PlanKind) for B transforms of a plan per block of 256 lanes.
+int plan_kind(const FftPlan &p, int B);
 // Standalone batched 2D FFT (in place).
 void launch_fft2(float2 *data, const FftPlan &pw, const FftPlan &ph, int H, int W, int batch,
                  int sign, int centered, float scale, hipStream_t s);

@@ -282,8 +282,7 @@ void launch_compact_gather(const CartGeom &g, const float2 *dense, float2 *compa
   AV_LAUNCH_CHECK();
 }
 
-// fft_io's kind for B transforms of a plan per block.
-static int plan_kind(const FftPlan &p, int B) {
+int plan_kind(const FftPlan &p, int B) {
   if (p.ra && B * p.ra <= NT) return kPlanTwo;
   return plan_is_wide(p) ? kPlanWide : kPlanNarrow;
 }
