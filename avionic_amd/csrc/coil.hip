@@ -14,9 +14,8 @@
 //      quadratically regularised fit (B1Recon :217-362);
 //   4. a final B1Recon over all coils (:553-556).
 // Images are [coils][height][width] complex float; arithmetic is float (the
-// reference's precision), reductions are double in a fixed order.  Each PD
-// iteration is two fused kernels (dual ascent + projection, primal descent +
-// extragradient) over all pixels (and coils).
+// reference's precision), reductions are double in a fixed order.  The PD loops
+// run several iterations per launch on regions held in LDS.
 #include <algorithm>
 #include <cmath>
 #include <memory>
@@ -31,24 +30,6 @@ namespace {
 constexpr int kTC = 256;
 
 inline unsigned nblocks(long n) { return (unsigned)std::max<long>(1, std::min<long>(4096, (n + kTC - 1) / kTC)); }
-
-// Non-periodic 2D differences (utils::Gradient2D / Divergence2D etc.).
-__device__ inline float2 fdx(const float2 *a, int i, int x, int W) { return x < W - 1 ? csub(a[i + 1], a[i]) : czero(); }
-__device__ inline float2 fdy(const float2 *a, int i, int y, int W, int H) {
-  return y < H - 1 ? csub(a[i + W], a[i]) : czero();
-}
-__device__ inline float2 bdx(const float2 *a, int i, int x, int W) {
-  if (W == 1) return czero();
-  if (x == 0) return a[i];
-  if (x == W - 1) return cscale(a[i - 1], -1.f);
-  return csub(a[i], a[i - 1]);
-}
-__device__ inline float2 bdy(const float2 *a, int i, int y, int W, int H) {
-  if (H == 1) return czero();
-  if (y == 0) return a[i];
-  if (y == H - 1) return cscale(a[i - W], -1.f);
-  return csub(a[i], a[i - W]);
-}
 
 // ------------------------------------------------------------ time average
 // davg[c] = sum_t d[t][c] / max(1, sum_t M_t), mask from the compact rows.
@@ -131,103 +112,115 @@ __global__ void k_abs_max(const float2 *__restrict__ a, long N, double *__restri
 
 // ------------------------------------------------------------- B1FromUH1
 // Batched CG over the coils: A = diag(mu |u|^2) + L, L the periodic 2D
-// Laplacian (D^T D with wrap-around forward differences).
+// Laplacian (D^T D with wrap-around forward differences).  Images of this size
+// are bound by launches, so an iteration is two kernels: the direction update
+// and A p (the neighbours' new directions are recomputed), and the step.  Each
+// block sums the other kernel's block partials itself, in one fixed order; the
+// scalars alternate between two slots, written by block 0 of a coil.
 struct CgScal {
-  double rho, rho0, alpha;
+  double rho, rho0;
   int active;
 };
+// Sum of n <= kTC partials, in every lane.
+__device__ inline double sum_partials(const double *p, int n) {
+  __shared__ double red[kTC];
+  red[threadIdx.x] = (int)threadIdx.x < n ? p[threadIdx.x] : 0.0;
+  __syncthreads();
+  for (int s = kTC / 2; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  const double v = red[0];
+  __syncthreads();
+  return v;
+}
+// x = 0, p = 0, r = conj(u) mu |crec|; partial = sum |r|^2
 __global__ void k_cg_init(const float2 *__restrict__ u, const float2 *__restrict__ crec, float mu,
                           float2 *__restrict__ x, float2 *__restrict__ r, float2 *__restrict__ p,
-                          long N, int C) {
-  const long n = N * C;
-  for (long e = (long)blockIdx.x * kTC + threadIdx.x; e < n; e += (long)gridDim.x * kTC) {
-    const long i = e % N;
+                          long N, double *__restrict__ partial) {
+  const int c = blockIdx.y, nb = gridDim.x;
+  double acc = 0.0;
+  for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)nb * kTC) {
+    const long e = c * N + i;
     const float a = mu * sqrtf(cabs2(crec[e]));
     const float2 uu = u[i];
-    const float2 rhs = make_float2(uu.x * a, -uu.y * a);  // conj(u) mu |crec|
+    const float2 rhs = make_float2(uu.x * a, -uu.y * a);
     x[e] = czero();
+    p[e] = czero();
     r[e] = rhs;
-    p[e] = rhs;
+    acc += (double)cabs2(rhs);
   }
+  block_sum_store(acc, partial + (long)c * nb + blockIdx.x);
 }
-__device__ inline float2 lap_periodic(const float2 *a, int x, int y, int W, int H) {
-  const int i = y * W + x;
-  const int xp = x + 1 < W ? x + 1 : 0, xm = x > 0 ? x - 1 : W - 1;
-  const int yp = y + 1 < H ? y + 1 : 0, ym = y > 0 ? y - 1 : H - 1;
-  const float2 c = a[i];
-  const float2 bx = cadd(csub(a[y * W + xp], cscale(c, 2.f)), a[y * W + xm]);
-  const float2 by = cadd(csub(a[yp * W + x], cscale(c, 2.f)), a[ym * W + x]);
-  return cscale(cadd(bx, by), -1.f);
-}
-// Ap = (mu |u|^2 + L) p for active coils; partial[c][b] = sum Re(conj(p) Ap)
-__global__ void k_cg_apply(const float2 *__restrict__ u, float mu, const float2 *__restrict__ p,
-                           float2 *__restrict__ ap, const CgScal *__restrict__ sc, int W, int H,
-                           double *__restrict__ partial) {
+// Convergence (squared residual <= 1e-12 rho0 or <= 1e-12), then for active
+// coils p' = r + beta p and Ap = (mu |u|^2 + L) p'; pap = sum Re(conj(p') Ap).
+// rr: block partials of |r|^2; first: the first iteration (rho0 = |r|^2,
+// beta = 0).
+__global__ __launch_bounds__(kTC) void k_cg_apply(const float2 *__restrict__ u, float mu,
+                                                  const float2 *__restrict__ r,
+                                                  const float2 *__restrict__ pin,
+                                                  float2 *__restrict__ pout,
+                                                  float2 *__restrict__ ap,
+                                                  const CgScal *__restrict__ sin,
+                                                  CgScal *__restrict__ sout, int first, int W,
+                                                  int H, const double *__restrict__ rr,
+                                                  double *__restrict__ pap) {
   const int c = blockIdx.y, nb = gridDim.x;
   const long N = (long)W * H;
+  const double rn = sum_partials(rr + (long)c * nb, nb);
+  CgScal s = sin[c];
+  double beta = 0.0;
+  if (first) {
+    s.rho = s.rho0 = rn;
+    s.active = rn > 1e-12 ? 1 : 0;
+  } else if (s.active) {
+    if (rn <= 1e-12 * s.rho0 || rn <= 1e-12) {
+      s.active = 0;
+    } else {
+      beta = rn / s.rho;
+      s.rho = rn;
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) sout[c] = s;
   double acc = 0.0;
-  if (sc[c].active) {
-    const float2 *pc = p + c * N;
+  if (s.active) {
+    const float be = (float)beta;
+    const float2 *rc = r + c * N, *pc = pin + c * N;
+    auto dir = [&](int i) { return cadd(rc[i], cscale(pc[i], be)); };
     for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)nb * kTC) {
       const int x = (int)(i % W), y = (int)(i / W);
-      const float2 v = cadd(lap_periodic(pc, x, y, W, H), cscale(pc[i], mu * cabs2(u[i])));
+      const int xp = x + 1 < W ? x + 1 : 0, xm = x > 0 ? x - 1 : W - 1;
+      const int yp = y + 1 < H ? y + 1 : 0, ym = y > 0 ? y - 1 : H - 1;
+      const float2 pv = dir((int)i);
+      const float2 bx = cadd(csub(dir(y * W + xp), cscale(pv, 2.f)), dir(y * W + xm));
+      const float2 by = cadd(csub(dir(yp * W + x), cscale(pv, 2.f)), dir(ym * W + x));
+      const float2 v = cadd(cscale(cadd(bx, by), -1.f), cscale(pv, mu * cabs2(u[i])));
+      pout[c * N + i] = pv;
       ap[c * N + i] = v;
-      acc += (double)pc[i].x * v.x + (double)pc[i].y * v.y;
+      acc += (double)pv.x * v.x + (double)pv.y * v.y;
     }
   }
-  block_sum_store(acc, partial + (long)c * nb + blockIdx.x);
+  block_sum_store(acc, pap + (long)c * nb + blockIdx.x);
 }
-// alpha = rho / <p, Ap>
-__global__ void k_cg_alpha(CgScal *sc, const double *__restrict__ partial, int nb) {
-  const int c = blockIdx.x;
-  if (threadIdx.x != 0 || !sc[c].active) return;
-  double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += partial[(long)c * nb + b];
-  sc[c].alpha = sc[c].rho / s;
-}
-// x += alpha p; r -= alpha Ap; partial = sum |r|^2
-__global__ void k_cg_update(float2 *__restrict__ x, float2 *__restrict__ r,
-                            const float2 *__restrict__ p, const float2 *__restrict__ ap,
-                            const CgScal *__restrict__ sc, long N, double *__restrict__ partial) {
+// alpha = rho / <p, Ap>; x += alpha p; r -= alpha Ap; rr = sum |r|^2
+__global__ __launch_bounds__(kTC) void k_cg_update(float2 *__restrict__ x, float2 *__restrict__ r,
+                                                   const float2 *__restrict__ p,
+                                                   const float2 *__restrict__ ap,
+                                                   const CgScal *__restrict__ sc, long N,
+                                                   const double *__restrict__ pap,
+                                                   double *__restrict__ rr) {
   const int c = blockIdx.y, nb = gridDim.x;
+  if (!sc[c].active) return;
+  const float al = (float)(sc[c].rho / sum_partials(pap + (long)c * nb, nb));
   double acc = 0.0;
-  if (sc[c].active) {
-    const float al = (float)sc[c].alpha;
-    for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)nb * kTC) {
-      const long e = c * N + i;
-      x[e] = cadd(x[e], cscale(p[e], al));
-      const float2 rn = csub(r[e], cscale(ap[e], al));
-      r[e] = rn;
-      acc += (double)cabs2(rn);
-    }
-  }
-  block_sum_store(acc, partial + (long)c * nb + blockIdx.x);
-}
-// convergence (squared residual <= 1e-12 rho0 or <= 1e-12) and beta
-__global__ void k_cg_beta(CgScal *sc, const double *__restrict__ partial, int nb, double *beta) {
-  const int c = blockIdx.x;
-  if (threadIdx.x != 0) return;
-  beta[c] = 0.0;
-  if (!sc[c].active) return;
-  double rn = 0.0;
-  for (int b = 0; b < nb; ++b) rn += partial[(long)c * nb + b];
-  if (rn <= 1e-12 * sc[c].rho0 || rn <= 1e-12) {
-    sc[c].active = 0;
-    return;
-  }
-  beta[c] = rn / sc[c].rho;
-  sc[c].rho = rn;
-}
-__global__ void k_cg_direction(float2 *__restrict__ p, const float2 *__restrict__ r,
-                               const CgScal *__restrict__ sc, const double *__restrict__ beta,
-                               long N) {
-  const int c = blockIdx.y;
-  if (!sc[c].active) return;
-  const float be = (float)beta[c];
-  for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)gridDim.x * kTC) {
+  for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)nb * kTC) {
     const long e = c * N + i;
-    p[e] = cadd(r[e], cscale(p[e], be));
+    x[e] = cadd(x[e], cscale(p[e], al));
+    const float2 rn = csub(r[e], cscale(ap[e], al));
+    r[e] = rn;
+    acc += (double)cabs2(rn);
   }
+  block_sum_store(acc, rr + (long)c * nb + blockIdx.x);
 }
 // b1_c = |x_c| / sqrt(sum_c |x_c|^2)
 __global__ void k_cg_finish(const float2 *__restrict__ x, float2 *__restrict__ b1, int C, long N) {
@@ -256,105 +249,255 @@ __global__ void k_ut_pre(const float2 *__restrict__ b1, const float2 *__restrict
     ib[i] = 1.f / (1.f + tau * s);
   }
 }
-struct UtState {
-  float2 *x1, *ext1, *x2, *ext2, *y1, *y2;  // x2 / ext2 / y1: 2 N, y2: 3 N
+// Several iterations of a PD loop per launch: a block holds a REG x REG region
+// in LDS and advances it `its` <= kHalo iterations.  An iteration reaches one
+// pixel in each direction, so after them the inner CORE x CORE pixels are the
+// ones the whole image would have given; the block writes those to the other
+// half of a double buffer.  The loops were bound by launches (4 us each, two per
+// iteration): coil estimation at 192 x 160, 12 frames, 6 coils, 38 -> 11
+// ms (the two-kernel conjugate gradients above included).
+constexpr int kHalo = 8;
+// Region side REG, lanes per block, pixels per lane (ROW rows apart).
+template <int REG_>
+struct Region {
+  static constexpr int REG = REG_, CORE = REG - 2 * kHalo, LANES = REG == 32 ? 1024 : 768,
+                       PIX = REG * REG / LANES, ROW = LANES / REG;
 };
-// y1 += sigma (grad ext1 - ext2); y2 += sigma E ext2; projections (radii
-// alpha1 nu and alpha0 nu; |y2| with the off-diagonal weight 2)
-__global__ void k_ut_dual(UtState s, int W, int H, float sigma, float r1, float r2) {
-  const long N = (long)W * H;
-  for (long e = (long)blockIdx.x * kTC + threadIdx.x; e < N; e += (long)gridDim.x * kTC) {
-    const int i = (int)e, x = i % W, y = i / W;
-    const float2 *v0 = s.ext2, *v1 = s.ext2 + N;
-    float2 p0 = cadd(s.y1[i], cscale(csub(fdx(s.ext1, i, x, W), v0[i]), sigma));
-    float2 p1 = cadd(s.y1[N + i], cscale(csub(fdy(s.ext1, i, y, W, H), v1[i]), sigma));
-    const float2 e0 = bdx(v0, i, x, W), e1 = bdy(v1, i, y, W, H);
-    const float2 e2 = cscale(cadd(bdy(v0, i, y, W, H), bdx(v1, i, x, W)), 0.5f);
-    float2 q0 = cadd(s.y2[i], cscale(e0, sigma));
-    float2 q1 = cadd(s.y2[N + i], cscale(e1, sigma));
-    float2 q2 = cadd(s.y2[2 * N + i], cscale(e2, sigma));
-    const float s1 = fmaxf(1.f, sqrtf(cabs2(p0) + cabs2(p1)) / r1);
-    const float s2 = fmaxf(1.f, sqrtf(cabs2(q0) + cabs2(q1) + 2.f * cabs2(q2)) / r2);
-    s.y1[i] = cscale(p0, 1.f / s1);
-    s.y1[N + i] = cscale(p1, 1.f / s1);
-    s.y2[i] = cscale(q0, 1.f / s2);
-    s.y2[N + i] = cscale(q1, 1.f / s2);
-    s.y2[2 * N + i] = cscale(q2, 1.f / s2);
+
+// A lane's k-th pixel: its place l in the region and i in the image.
+template <class G>
+struct RegPix {
+  int l, x, y, i;
+  bool in, core;
+  __device__ RegPix(int k, int W, int H) {
+    const int lx = (int)threadIdx.x % G::REG, ly = (int)threadIdx.x / G::REG + k * G::ROW;
+    l = ly * G::REG + lx;
+    x = (int)blockIdx.x * G::CORE - kHalo + lx;
+    y = (int)blockIdx.y * G::CORE - kHalo + ly;
+    in = x >= 0 && x < W && y >= 0 && y < H;
+    i = in ? y * W + x : 0;
+    core = in && lx >= kHalo && lx < G::REG - kHalo && ly >= kHalo && ly < G::REG - kHalo;
   }
-}
-// x1+ = (x1 + tau div y1 + tau Lw) ib; x2+ = x2 + tau (y1 + divsym y2);
-// ext = 2 x+ - x; x = x+
-__global__ void k_ut_primal(UtState s, const float2 *__restrict__ lw, const float *__restrict__ ib,
-                            int W, int H, float tau) {
+};
+// Differences on the region; a neighbour outside it (clamped) only reaches
+// pixels that the launch does not write.
+template <class G>
+struct RegDiff {
+  int W, H;
+  __device__ float2 at(const float2 *a, int l) const { return a[min(max(l, 0), G::REG * G::REG - 1)]; }
+  __device__ float2 fx(const float2 *a, const RegPix<G> &p, float2 c) const {
+    return p.x < W - 1 ? csub(at(a, p.l + 1), c) : czero();
+  }
+  __device__ float2 fy(const float2 *a, const RegPix<G> &p, float2 c) const {
+    return p.y < H - 1 ? csub(at(a, p.l + G::REG), c) : czero();
+  }
+  __device__ float2 bx(const float2 *a, const RegPix<G> &p, float2 c) const {
+    if (W == 1) return czero();
+    if (p.x == 0) return c;
+    const float2 m = at(a, p.l - 1);
+    return p.x == W - 1 ? cscale(m, -1.f) : csub(c, m);
+  }
+  __device__ float2 by(const float2 *a, const RegPix<G> &p, float2 c) const {
+    if (H == 1) return czero();
+    if (p.y == 0) return c;
+    const float2 m = at(a, p.l - G::REG);
+    return p.y == H - 1 ? cscale(m, -1.f) : csub(c, m);
+  }
+};
+
+// x1, ext1, x2 (2), ext2 (2), y1 (2), y2 (3): N elements each
+constexpr int kUtState = 11;
+template <class G>
+__global__ __launch_bounds__(G::LANES) void k_ut_iterations(const float2 *__restrict__ in,
+                                                            float2 *__restrict__ out,
+                                                            const float2 *__restrict__ lw,
+                                                            const float *__restrict__ ib, int W,
+                                                            int H, float sigma, float tau, float r1,
+                                                            float r2, int its) {
+  extern __shared__ float2 sh[];  // ext1, ext2 (2), y1 (2), y2 (3)
+  constexpr int A = G::REG * G::REG;
+  float2 *e1 = sh, *v0 = sh + A, *v1 = sh + 2 * A, *p0 = sh + 3 * A, *p1 = sh + 4 * A,
+         *q0 = sh + 5 * A, *q1 = sh + 6 * A, *q2 = sh + 7 * A;
   const long N = (long)W * H;
-  for (long e = (long)blockIdx.x * kTC + threadIdx.x; e < N; e += (long)gridDim.x * kTC) {
-    const int i = (int)e, x = i % W, y = i / W;
-    const float2 *y10 = s.y1, *y11 = s.y1 + N, *q0 = s.y2, *q1 = s.y2 + N, *q2 = s.y2 + 2 * N;
-    const float2 dv = cadd(bdx(y10, i, x, W), bdy(y11, i, y, W, H));
-    const float2 sd0 = cadd(fdx(q0, i, x, W), fdy(q2, i, y, W, H));
-    const float2 sd1 = cadd(fdx(q2, i, x, W), fdy(q1, i, y, W, H));
-    const float2 xo = s.x1[i];
-    const float2 xn = cscale(cadd(cadd(xo, cscale(dv, tau)), cscale(lw[i], tau)), ib[i]);
-    s.ext1[i] = csub(cscale(xn, 2.f), xo);
-    s.x1[i] = xn;
-    const float2 a0 = s.x2[i], a1 = s.x2[N + i];
-    const float2 n0 = cadd(a0, cscale(cadd(y10[i], sd0), tau));
-    const float2 n1 = cadd(a1, cscale(cadd(y11[i], sd1), tau));
-    s.ext2[i] = csub(cscale(n0, 2.f), a0);
-    s.ext2[N + i] = csub(cscale(n1, 2.f), a1);
-    s.x2[i] = n0;
-    s.x2[N + i] = n1;
+  const RegDiff<G> d{W, H};
+  float2 x1[G::PIX], xa[G::PIX], xb[G::PIX], l[G::PIX];
+  float b[G::PIX];
+#pragma unroll
+  for (int k = 0; k < G::PIX; ++k) {
+    const RegPix<G> p(k, W, H);
+    auto ld = [&](int c) { return p.in ? in[c * N + p.i] : czero(); };
+    x1[k] = ld(0);
+    xa[k] = ld(2);
+    xb[k] = ld(3);
+    l[k] = p.in ? lw[p.i] : czero();
+    b[k] = p.in ? ib[p.i] : 0.f;
+    e1[p.l] = ld(1);
+    v0[p.l] = ld(4);
+    v1[p.l] = ld(5);
+    p0[p.l] = ld(6);
+    p1[p.l] = ld(7);
+    q0[p.l] = ld(8);
+    q1[p.l] = ld(9);
+    q2[p.l] = ld(10);
+  }
+  __syncthreads();
+  for (int it = 0; it < its; ++it) {
+    // y1 += sigma (grad ext1 - ext2); y2 += sigma E ext2; projections (radii
+    // alpha1 nu and alpha0 nu; |y2| with the off-diagonal weight 2)
+#pragma unroll
+    for (int k = 0; k < G::PIX; ++k) {
+      const RegPix<G> p(k, W, H);
+      const float2 e = e1[p.l], a = v0[p.l], c = v1[p.l];
+      const float2 s0 = cadd(p0[p.l], cscale(csub(d.fx(e1, p, e), a), sigma));
+      const float2 s1 = cadd(p1[p.l], cscale(csub(d.fy(e1, p, e), c), sigma));
+      const float2 g2 = cscale(cadd(d.by(v0, p, a), d.bx(v1, p, c)), 0.5f);
+      const float2 t0 = cadd(q0[p.l], cscale(d.bx(v0, p, a), sigma));
+      const float2 t1 = cadd(q1[p.l], cscale(d.by(v1, p, c), sigma));
+      const float2 t2 = cadd(q2[p.l], cscale(g2, sigma));
+      const float n1 = fmaxf(1.f, sqrtf(cabs2(s0) + cabs2(s1)) / r1);
+      const float n2 = fmaxf(1.f, sqrtf(cabs2(t0) + cabs2(t1) + 2.f * cabs2(t2)) / r2);
+      p0[p.l] = cscale(s0, 1.f / n1);
+      p1[p.l] = cscale(s1, 1.f / n1);
+      q0[p.l] = cscale(t0, 1.f / n2);
+      q1[p.l] = cscale(t1, 1.f / n2);
+      q2[p.l] = cscale(t2, 1.f / n2);
+    }
+    __syncthreads();
+    // x1+ = (x1 + tau div y1 + tau Lw) ib; x2+ = x2 + tau (y1 + divsym y2);
+    // ext = 2 x+ - x; x = x+
+#pragma unroll
+    for (int k = 0; k < G::PIX; ++k) {
+      const RegPix<G> p(k, W, H);
+      const float2 a = p0[p.l], c = p1[p.l], t0 = q0[p.l], t1 = q1[p.l], t2 = q2[p.l];
+      const float2 dv = cadd(d.bx(p0, p, a), d.by(p1, p, c));
+      const float2 sd0 = cadd(d.fx(q0, p, t0), d.fy(q2, p, t2));
+      const float2 sd1 = cadd(d.fx(q2, p, t2), d.fy(q1, p, t1));
+      const float2 xn = cscale(cadd(cadd(x1[k], cscale(dv, tau)), cscale(l[k], tau)), b[k]);
+      const float2 n0 = cadd(xa[k], cscale(cadd(a, sd0), tau));
+      const float2 n1 = cadd(xb[k], cscale(cadd(c, sd1), tau));
+      e1[p.l] = csub(cscale(xn, 2.f), x1[k]);
+      v0[p.l] = csub(cscale(n0, 2.f), xa[k]);
+      v1[p.l] = csub(cscale(n1, 2.f), xb[k]);
+      x1[k] = xn;
+      xa[k] = n0;
+      xb[k] = n1;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < G::PIX; ++k) {
+    const RegPix<G> p(k, W, H);
+    if (!p.core) continue;
+    auto st = [&](int c, float2 v) { out[c * N + p.i] = v; };
+    st(0, x1[k]);
+    st(1, e1[p.l]);
+    st(2, xa[k]);
+    st(3, xb[k]);
+    st(4, v0[p.l]);
+    st(5, v1[p.l]);
+    st(6, p0[p.l]);
+    st(7, p1[p.l]);
+    st(8, q0[p.l]);
+    st(9, q1[p.l]);
+    st(10, q2[p.l]);
   }
 }
 
 // --------------------------------------------------------------- B1Recon
-// un = u0 / max|u0|: lw_c = conj(un) crec_c, iu = 1 / (1 + tau |un|^2)
-__global__ void k_b1_pre(const float2 *__restrict__ u0, const float2 *__restrict__ crec,
-                         const double *__restrict__ mx, float tau, int coils, long N,
-                         float2 *__restrict__ lw, float *__restrict__ iu) {
-  const float inv = (float)(1.0 / *mx);
+// un = u0 / max|u0|: lw_c = conj(un) crec_c, iu = 1 / (1 + tau |un|^2); the
+// maximum from nmx <= kTC block partials, stored at *mx
+__global__ __launch_bounds__(kTC) void k_b1_pre(const float2 *__restrict__ u0,
+                                                const float2 *__restrict__ crec,
+                                                const double *__restrict__ part, int nmx,
+                                                double *__restrict__ mx, float tau, int coils,
+                                                long N, float2 *__restrict__ lw,
+                                                float *__restrict__ iu) {
+  __shared__ double red[kTC];
+  red[threadIdx.x] = (int)threadIdx.x < nmx ? part[threadIdx.x] : 0.0;
+  __syncthreads();
+  for (int s = kTC / 2; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
+    __syncthreads();
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *mx = red[0];
+  const float inv = (float)(1.0 / red[0]);
   for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)gridDim.x * kTC) {
     const float2 un = cscale(u0[i], inv);
     iu[i] = 1.f / (1.f + tau * cabs2(un));
     for (int c = 0; c < coils; ++c) lw[c * N + i] = cmulc(un, crec[c * N + i]);
   }
 }
-// y_c = (y_c + sigma grad ext_c) / (1 + sigma / mu)
-__global__ void k_b1_dual(const float2 *__restrict__ ext, float2 *__restrict__ y, int W, int H,
-                          int coils, float sigma, float shrink) {
-  const long N = (long)W * H, n = N * coils;
-  for (long e = (long)blockIdx.x * kTC + threadIdx.x; e < n; e += (long)gridDim.x * kTC) {
-    const long c = e / N;
-    const int i = (int)(e % N), x = i % W, y0 = i / W;
-    const float2 *ec = ext + c * N;
-    float2 *yc = y + 2 * c * N;
-    yc[i] = cscale(cadd(yc[i], cscale(fdx(ec, i, x, W), sigma)), shrink);
-    yc[N + i] = cscale(cadd(yc[N + i], cscale(fdy(ec, i, y0, W, H), sigma)), shrink);
+// Iterations of one coil (blockIdx.z) on the region form above; a coil's state
+// is x, ext, y (2): N elements each.
+//   y = (y + sigma grad ext) / (1 + sigma / mu)
+//   x+ = (x + tau div y + tau lw) iu; ext = 2 x+ - x; x = x+
+constexpr int kB1State = 4;
+template <class G>
+__global__ __launch_bounds__(G::LANES) void k_b1_iterations(const float2 *__restrict__ in,
+                                                            float2 *__restrict__ out,
+                                                            const float2 *__restrict__ lw,
+                                                            const float *__restrict__ iu, int W,
+                                                            int H, float sigma, float shrink,
+                                                            float tau, int its) {
+  __shared__ float2 e1[G::REG * G::REG], y0[G::REG * G::REG], y1[G::REG * G::REG];
+  const long N = (long)W * H;
+  const RegDiff<G> d{W, H};
+  in += (long)blockIdx.z * kB1State * N;
+  out += (long)blockIdx.z * kB1State * N;
+  lw += (long)blockIdx.z * N;
+  float2 x[G::PIX], ext[G::PIX], a[G::PIX], c[G::PIX], l[G::PIX];
+  float b[G::PIX];
+#pragma unroll
+  for (int k = 0; k < G::PIX; ++k) {
+    const RegPix<G> p(k, W, H);
+    x[k] = p.in ? in[p.i] : czero();
+    ext[k] = p.in ? in[N + p.i] : czero();
+    a[k] = p.in ? in[2 * N + p.i] : czero();
+    c[k] = p.in ? in[3 * N + p.i] : czero();
+    l[k] = p.in ? lw[p.i] : czero();
+    b[k] = p.in ? iu[p.i] : 0.f;
+    e1[p.l] = ext[k];
+  }
+  __syncthreads();
+  for (int it = 0; it < its; ++it) {
+#pragma unroll
+    for (int k = 0; k < G::PIX; ++k) {
+      const RegPix<G> p(k, W, H);
+      a[k] = cscale(cadd(a[k], cscale(d.fx(e1, p, ext[k]), sigma)), shrink);
+      c[k] = cscale(cadd(c[k], cscale(d.fy(e1, p, ext[k]), sigma)), shrink);
+      y0[p.l] = a[k];
+      y1[p.l] = c[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < G::PIX; ++k) {
+      const RegPix<G> p(k, W, H);
+      const float2 dv = cadd(d.bx(y0, p, a[k]), d.by(y1, p, c[k]));
+      const float2 xn = cscale(cadd(cadd(x[k], cscale(dv, tau)), cscale(l[k], tau)), b[k]);
+      ext[k] = csub(cscale(xn, 2.f), x[k]);
+      x[k] = xn;
+      e1[p.l] = ext[k];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < G::PIX; ++k) {
+    const RegPix<G> p(k, W, H);
+    if (!p.core) continue;
+    out[p.i] = x[k];
+    out[N + p.i] = ext[k];
+    out[2 * N + p.i] = a[k];
+    out[3 * N + p.i] = c[k];
   }
 }
-// x+ = (x + tau div y_c + tau lw_c) iu; ext = 2 x+ - x; x = x+
-__global__ void k_b1_primal(float2 *__restrict__ x1, float2 *__restrict__ ext,
-                            const float2 *__restrict__ y, const float2 *__restrict__ lw,
-                            const float *__restrict__ iu, int W, int H, int coils, float tau) {
-  const long N = (long)W * H, n = N * coils;
-  for (long e = (long)blockIdx.x * kTC + threadIdx.x; e < n; e += (long)gridDim.x * kTC) {
-    const long c = e / N;
-    const int i = (int)(e % N), x = i % W, y0 = i / W;
-    const float2 *yc = y + 2 * c * N;
-    const float2 dv = cadd(bdx(yc, i, x, W), bdy(yc + N, i, y0, W, H));
-    const float2 xo = x1[e];
-    const float2 xn = cscale(cadd(cadd(xo, cscale(dv, tau)), cscale(lw[e], tau)), iu[i]);
-    ext[e] = csub(cscale(xn, 2.f), xo);
-    x1[e] = xn;
-  }
-}
-// x_c /= sqrt(sum_c |x_c|^2)
-__global__ void k_b1_normalize(float2 *__restrict__ x, int coils, long N) {
+// x_c = s_c / sqrt(sum_c |s_c|^2) from the coils' states
+__global__ void k_b1_normalize(const float2 *__restrict__ s, float2 *__restrict__ x, int coils,
+                               long N) {
   for (long i = (long)blockIdx.x * kTC + threadIdx.x; i < N; i += (long)gridDim.x * kTC) {
-    float s = 0.f;
-    for (int c = 0; c < coils; ++c) s += cabs2(x[c * N + i]);
-    const float inv = 1.f / sqrtf(s);
-    for (int c = 0; c < coils; ++c) x[c * N + i] = cscale(x[c * N + i], inv);
+    float m = 0.f;
+    for (int c = 0; c < coils; ++c) m += cabs2(s[c * kB1State * N + i]);
+    const float inv = 1.f / sqrtf(m);
+    for (int c = 0; c < coils; ++c) x[c * N + i] = cscale(s[c * kB1State * N + i], inv);
   }
 }
 
@@ -380,15 +523,6 @@ __global__ void k_apply_phase(const float2 *__restrict__ absb, const float2 *__r
     const float ph = atan2f(x[i].y, x[i].x);
     out[i] = cmul(absb[i], make_float2(cosf(ph), sinf(ph)));
   }
-}
-
-double host_sum(const double *d, long n, hipStream_t s, long stride = 1, long off = 0) {
-  std::vector<double> h((size_t)n * stride);
-  AV_HIP(hipMemcpyAsync(h.data(), d, sizeof(double) * h.size(), hipMemcpyDeviceToHost, s));
-  AV_HIP(hipStreamSynchronize(s));
-  double a = 0.0;
-  for (long k = 0; k < n; ++k) a += h[(size_t)(k * stride + off)];
-  return a;
 }
 
 }  // namespace
@@ -474,53 +608,32 @@ void coil_time_averaged(const Operator &op, const float2 *kdata, float2 *u, floa
 void coil_b1_from_uh1(const CoilCtx &k, const float2 *u, const float2 *crec, double mu,
                       float2 *b1) {
   const long n = k.N * k.C;
-  DevBuf x, r, p, ap, sc, part, beta;
+  DevBuf x, r, p, ap, sc, part;
   x.ensure(sizeof(float2) * n);
   r.ensure(sizeof(float2) * n);
-  p.ensure(sizeof(float2) * n);
+  p.ensure(sizeof(float2) * 2 * n);
   ap.ensure(sizeof(float2) * n);
-  sc.ensure(sizeof(CgScal) * k.C);
-  beta.ensure(sizeof(double) * k.C);
-  const int nb = (int)std::min<long>(256, (k.N + kTC - 1) / kTC);
-  part.ensure(sizeof(double) * (size_t)nb * k.C);
-  hipLaunchKernelGGL(k_cg_init, dim3(nblocks(n)), dim3(kTC), 0, k.s, u, crec, (float)mu,
-                     x.as<float2>(), r.as<float2>(), p.as<float2>(), k.N, k.C);
-  AV_LAUNCH_CHECK();
-  // rho0 = |r|^2 per coil
-  {
-    std::vector<CgScal> hs(k.C);
-    const float2 *rr = r.as<float2>();
-    std::vector<float2> hr((size_t)n);
-    AV_HIP(hipMemcpyAsync(hr.data(), rr, sizeof(float2) * n, hipMemcpyDeviceToHost, k.s));
-    AV_HIP(hipStreamSynchronize(k.s));
-    for (int c = 0; c < k.C; ++c) {
-      double a = 0.0;
-      for (long i = 0; i < k.N; ++i) {
-        const float2 v = hr[(size_t)(c * k.N + i)];
-        a += (double)v.x * v.x + (double)v.y * v.y;
-      }
-      hs[c].rho = hs[c].rho0 = a;
-      hs[c].alpha = 0.0;
-      hs[c].active = a > 1e-12 ? 1 : 0;
-    }
-    AV_HIP(hipMemcpyAsync(sc.p, hs.data(), sizeof(CgScal) * k.C, hipMemcpyHostToDevice, k.s));
-  }
+  sc.ensure(sizeof(CgScal) * 2 * k.C);
+  const int nb = (int)std::min<long>(kTC, (k.N + kTC - 1) / kTC);
+  part.ensure(sizeof(double) * 2 * (size_t)nb * k.C);
+  double *rr = part.as<double>(), *pap = rr + (size_t)nb * k.C;
+  float2 *pb[2] = {p.as<float2>(), p.as<float2>() + n};
+  CgScal *sb[2] = {sc.as<CgScal>(), sc.as<CgScal>() + k.C};
   const dim3 grid(nb, k.C);
+  AV_HIP(hipMemsetAsync(sc.p, 0, sc.bytes, k.s));
+  hipLaunchKernelGGL(k_cg_init, grid, dim3(kTC), 0, k.s, u, crec, (float)mu, x.as<float2>(),
+                     r.as<float2>(), pb[0], k.N, rr);
+  AV_LAUNCH_CHECK();
   for (int it = 0; it < 800; ++it) {
-    hipLaunchKernelGGL(k_cg_apply, grid, dim3(kTC), 0, k.s, u, (float)mu, p.as<float2>(),
-                       ap.as<float2>(), sc.as<CgScal>(), k.W, k.H, part.as<double>());
-    hipLaunchKernelGGL(k_cg_alpha, dim3(k.C), dim3(64), 0, k.s, sc.as<CgScal>(), part.as<double>(),
-                       nb);
-    hipLaunchKernelGGL(k_cg_update, grid, dim3(kTC), 0, k.s, x.as<float2>(), r.as<float2>(),
-                       p.as<float2>(), ap.as<float2>(), sc.as<CgScal>(), k.N, part.as<double>());
-    hipLaunchKernelGGL(k_cg_beta, dim3(k.C), dim3(64), 0, k.s, sc.as<CgScal>(), part.as<double>(),
-                       nb, beta.as<double>());
-    hipLaunchKernelGGL(k_cg_direction, grid, dim3(kTC), 0, k.s, p.as<float2>(), r.as<float2>(),
-                       sc.as<CgScal>(), beta.as<double>(), k.N);
+    const int a = it & 1, b = 1 - a;
+    hipLaunchKernelGGL(k_cg_apply, grid, dim3(kTC), 0, k.s, u, (float)mu, r.as<float2>(), pb[a],
+                       pb[b], ap.as<float2>(), sb[a], sb[b], it == 0 ? 1 : 0, k.W, k.H, rr, pap);
+    hipLaunchKernelGGL(k_cg_update, grid, dim3(kTC), 0, k.s, x.as<float2>(), r.as<float2>(), pb[b],
+                       ap.as<float2>(), sb[b], k.N, pap, rr);
     AV_LAUNCH_CHECK();
-    if ((it & 15) == 15) {  // stop once every coil has converged
+    if ((it & 15) == 0 && it > 0) {  // stop once every coil had converged before this iteration
       std::vector<CgScal> hs(k.C);
-      AV_HIP(hipMemcpyAsync(hs.data(), sc.p, sizeof(CgScal) * k.C, hipMemcpyDeviceToHost, k.s));
+      AV_HIP(hipMemcpyAsync(hs.data(), sb[b], sizeof(CgScal) * k.C, hipMemcpyDeviceToHost, k.s));
       AV_HIP(hipStreamSynchronize(k.s));
       bool any = false;
       for (const CgScal &c : hs) any = any || c.active;
@@ -532,6 +645,34 @@ void coil_b1_from_uh1(const CoilCtx &k, const float2 *u, const float2 *crec, dou
   AV_LAUNCH_CHECK();
 }
 
+template <class G>
+static dim3 region_grid(const CoilCtx &k, int coils) {
+  return dim3((k.W + G::CORE - 1) / G::CORE, (k.H + G::CORE - 1) / G::CORE, coils);
+}
+// Small regions (one pixel per lane, four times the core's pixels computed)
+// where they make at most four blocks per CU, large ones (2.25 times) above.
+// Measured on MI355X, large / small: one image of 192 x 160, 14.2 / 7.3 us per
+// launch of B1Recon iterations; whole estimation 192x160x6 14.7 / 11 ms, 256x256x8
+// 19.6 / 14.6 ms with small ones for the single images only.
+static bool small_regions(const CoilCtx &k, int coils) {
+  const dim3 g = region_grid<Region<32>>(k, coils);
+  return (long)g.x * g.y * g.z <= 1024;
+}
+template <class G>
+static void ut_iterations(const CoilCtx &k, const float2 *in, float2 *out, const float2 *lw,
+                          const float *ib, float sigma, float tau, float r1, float r2, int its) {
+  hipLaunchKernelGGL(k_ut_iterations<G>, region_grid<G>(k, 1), dim3(G::LANES),
+                     sizeof(float2) * 8 * G::REG * G::REG, k.s, in, out, lw, ib, k.W, k.H, sigma, tau,
+                     r1, r2, its);
+}
+template <class G>
+static void b1_iterations(const CoilCtx &k, int coils, const float2 *in, float2 *out,
+                          const float2 *lw, const float *iu, float sigma, float shrink, float tau,
+                          int its) {
+  hipLaunchKernelGGL(k_b1_iterations<G>, region_grid<G>(k, coils), dim3(G::LANES), 0, k.s, in, out,
+                     lw, iu, k.W, k.H, sigma, shrink, tau, its);
+}
+
 void coil_utgv2(const CoilCtx &k, const float2 *b1, const float2 *crec, const std::vector<int> &inds,
                 const avionic_coil_params &p, float2 *x_inout) {
   const long N = k.N;
@@ -540,67 +681,56 @@ void coil_utgv2(const CoilCtx &k, const float2 *b1, const float2 *crec, const st
   AV_HIP(hipMemcpyAsync(bi.p, inds.data(), sizeof(int) * inds.size(), hipMemcpyHostToDevice, k.s));
   lw.ensure(sizeof(float2) * N);
   ib.ensure(sizeof(float) * N);
-  st.ensure(sizeof(float2) * N * 10);  // ext1, x2 (2), ext2 (2), y1 (2), y2 (3)
-  AV_HIP(hipMemsetAsync(st.p, 0, st.bytes, k.s));
-  UtState s;
-  s.x1 = x_inout;
-  s.ext1 = st.as<float2>();
-  s.x2 = s.ext1 + N;
-  s.ext2 = s.x2 + 2 * N;
-  s.y1 = s.ext2 + 2 * N;
-  s.y2 = s.y1 + 2 * N;
-  AV_HIP(hipMemcpyAsync(s.ext1, x_inout, sizeof(float2) * N, hipMemcpyDeviceToDevice, k.s));
+  st.ensure(sizeof(float2) * N * kUtState * 2);
+  float2 *sb[2] = {st.as<float2>(), st.as<float2>() + N * kUtState};
+  AV_HIP(hipMemsetAsync(sb[0], 0, sizeof(float2) * N * kUtState, k.s));
+  for (int c = 0; c < 2; ++c)  // x1, ext1
+    AV_HIP(hipMemcpyAsync(sb[0] + c * N, x_inout, sizeof(float2) * N, hipMemcpyDeviceToDevice, k.s));
   const float tau = (float)p.uTau, sigma = (float)p.uSigma;
   hipLaunchKernelGGL(k_ut_pre, dim3(nblocks(N)), dim3(kTC), 0, k.s, b1, crec, bi.as<int>(),
                      (int)inds.size(), tau, N, lw.as<float2>(), ib.as<float>());
   AV_LAUNCH_CHECK();
   const float r1 = (float)(p.uAlpha1 * p.uReg), r2 = (float)(p.uAlpha0 * p.uReg);
-  for (unsigned it = 0; it < p.uNrIt; ++it) {
-    hipLaunchKernelGGL(k_ut_dual, dim3(nblocks(N)), dim3(kTC), 0, k.s, s, k.W, k.H, sigma, r1, r2);
-    hipLaunchKernelGGL(k_ut_primal, dim3(nblocks(N)), dim3(kTC), 0, k.s, s, lw.as<float2>(),
-                       ib.as<float>(), k.W, k.H, tau);
-  }
+  int cur = 0;
+  const auto iterate = small_regions(k, 1) ? ut_iterations<Region<32>> : ut_iterations<Region<48>>;
+  for (unsigned it = 0; it < p.uNrIt; it += kHalo, cur = 1 - cur)
+    iterate(k, sb[cur], sb[1 - cur], lw.as<float2>(), ib.as<float>(), sigma, tau, r1, r2,
+            (int)std::min<unsigned>(kHalo, p.uNrIt - it));
   AV_LAUNCH_CHECK();
+  AV_HIP(hipMemcpyAsync(x_inout, sb[cur], sizeof(float2) * N, hipMemcpyDeviceToDevice, k.s));
   AV_HIP(hipStreamSynchronize(k.s));  // the index table stays alive until here
 }
 
 void coil_b1_recon(const CoilCtx &k, const float2 *u0, const float2 *crec, int coils,
                    unsigned maxit, double mu, const avionic_coil_params &p, float2 *x1) {
   const long N = k.N, n = N * coils;
-  DevBuf ext, y, lw, iu, part;
-  ext.ensure(sizeof(float2) * n);
-  y.ensure(sizeof(float2) * 2 * n);
+  DevBuf st, lw, iu, part;
+  st.ensure(sizeof(float2) * n * kB1State * 2);
   lw.ensure(sizeof(float2) * n);
   iu.ensure(sizeof(float) * N);
-  const int nb = (int)std::min<long>(256, (N + kTC - 1) / kTC);
+  const int nb = (int)std::min<long>(kTC, (N + kTC - 1) / kTC);
   part.ensure(sizeof(double) * (nb + 1));
-  AV_HIP(hipMemsetAsync(x1, 0, sizeof(float2) * n, k.s));
-  AV_HIP(hipMemsetAsync(ext.p, 0, ext.bytes, k.s));
-  AV_HIP(hipMemsetAsync(y.p, 0, y.bytes, k.s));
+  float2 *sb[2] = {st.as<float2>(), st.as<float2>() + n * kB1State};
+  AV_HIP(hipMemsetAsync(sb[0], 0, sizeof(float2) * n * kB1State, k.s));
   hipLaunchKernelGGL(k_abs_max, dim3(nb), dim3(kTC), 0, k.s, u0, N, part.as<double>());
   AV_LAUNCH_CHECK();
-  std::vector<double> hm(nb);
-  AV_HIP(hipMemcpyAsync(hm.data(), part.p, sizeof(double) * nb, hipMemcpyDeviceToHost, k.s));
-  AV_HIP(hipStreamSynchronize(k.s));
-  double mx = 0.0;
-  for (double v : hm) mx = std::max(mx, v);
-  AV_CHECK(mx > 0.0, "coil construction: the image estimate is zero");
-  AV_HIP(hipMemcpyAsync(part.as<double>() + nb, &mx, sizeof(double), hipMemcpyHostToDevice, k.s));
   const float tau = (float)p.b1Tau, sigma = (float)p.b1Sigma;
-  hipLaunchKernelGGL(k_b1_pre, dim3(nblocks(N)), dim3(kTC), 0, k.s, u0, crec,
+  hipLaunchKernelGGL(k_b1_pre, dim3(nblocks(N)), dim3(kTC), 0, k.s, u0, crec, part.as<double>(), nb,
                      part.as<double>() + nb, tau, coils, N, lw.as<float2>(), iu.as<float>());
   AV_LAUNCH_CHECK();
   const float shrink = (float)(1.0 / (1.0 + p.b1Sigma / mu));
-  for (unsigned it = 0; it < maxit; ++it) {
-    hipLaunchKernelGGL(k_b1_dual, dim3(nblocks(n)), dim3(kTC), 0, k.s, ext.as<float2>(),
-                       y.as<float2>(), k.W, k.H, coils, sigma, shrink);
-    hipLaunchKernelGGL(k_b1_primal, dim3(nblocks(n)), dim3(kTC), 0, k.s, x1, ext.as<float2>(),
-                       y.as<float2>(), lw.as<float2>(), iu.as<float>(), k.W, k.H, coils, tau);
-  }
+  int cur = 0;
+  const auto iterate = small_regions(k, coils) ? b1_iterations<Region<32>> : b1_iterations<Region<48>>;
+  for (unsigned it = 0; it < maxit; it += kHalo, cur = 1 - cur)
+    iterate(k, coils, sb[cur], sb[1 - cur], lw.as<float2>(), iu.as<float>(), sigma, shrink, tau,
+            (int)std::min<unsigned>(kHalo, maxit - it));
   AV_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_b1_normalize, dim3(nblocks(N)), dim3(kTC), 0, k.s, x1, coils, N);
+  hipLaunchKernelGGL(k_b1_normalize, dim3(nblocks(N)), dim3(kTC), 0, k.s, sb[cur], x1, coils, N);
   AV_LAUNCH_CHECK();
-  AV_HIP(hipStreamSynchronize(k.s));  // `mx` is read by the copy above
+  double mx = 0.0;
+  AV_HIP(hipMemcpyAsync(&mx, part.as<double>() + nb, sizeof(double), hipMemcpyDeviceToHost, k.s));
+  AV_HIP(hipStreamSynchronize(k.s));
+  AV_CHECK(mx > 0.0, "coil construction: the image estimate is zero");
 }
 
 // PerformCoilConstruction (coil_construction.cpp:447-557) from the
