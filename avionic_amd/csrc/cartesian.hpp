@@ -70,9 +70,7 @@ class FftPlanCache;
 struct CartPlan {
   CartGeom g{};
   std::vector<int> h_row_off, h_rows;
-  void *d_row_off = nullptr, *d_rows = nullptr, *d_mrows = nullptr, *d_rowinfo = nullptr,
-       *d_rowmap = nullptr;
-  void *d_twx = nullptr, *d_twy = nullptr;
+  void *d_tables = nullptr;  // row_off, rows, rowinfo, rowmap, twiddles, mrows
   double mask_norm2 = 0.0;  // ||mask||^2 (AdaptLambda)
   bool has_mask = false;
 
@@ -104,6 +102,9 @@ inline int col_coil_groups(long tiles, int C) {
   return (int)std::min<long>(C, std::max<long>(1, 1024 / std::max<long>(1, tiles)));
 }
 
+// Radices of a length-L transform and its twiddles (tw[m] = exp(-2 pi i m / L))
+// on the host; make_fft_plan also uploads them.
+void fft_plan_host(int L, FftPlan &p, std::vector<float2> &tw);
 void make_fft_plan(int L, FftPlan &p, void **d_tw);
 
 // ---- launchers (all asynchronous on `s`) ----

@@ -40,7 +40,12 @@ struct Slot {
   std::unique_ptr<CartesianOperator> own_op;  // built from the request's mask
   Operator *op = nullptr;                     // the request's operator
   const CartesianOperator *cart = nullptr;    // op when it runs the task-list passes
-  DevBuf x, ext, y, z, d, khz, kcol, zhat, sc, slog, tlog, preg, pk, b1;
+  PoolBlock mem;  // every buffer below
+  hipStream_t busy = nullptr;  // stream of unfinished copies into them (submit)
+  ~Slot() {
+    if (busy) (void)hipStreamSynchronize(busy);
+  }
+  DevView x, ext, y, z, d, khz, kcol, zhat, sc, slog, tlog, preg, pk, b1;
   avionic_params params{};
   int maxit = 0, k_host = 0;
   bool done = false;
@@ -48,7 +53,7 @@ struct Slot {
   // in-loop PD gap (avionic_request_desc::verbose / debug, params.stopPDGap)
   bool verbose = false, debug = false;
   int debugstep = 1;
-  DevBuf gap_a, gap_b;
+  DevView gap_a, gap_b;
   std::vector<double> gap_log, norm_log, fid_log;
   size_t bytes = 0;
   Task task{};
@@ -121,6 +126,7 @@ struct Group {
 }  // namespace
 
 struct avionic_engine {
+  PoolUser pool_user;  // destroyed last: after the slots have given their blocks back
   // Every entry point taking an engine holds this for its whole call: calls
   // from several host threads are serialised (submit while another thread
   // steps or polls is safe).
@@ -487,7 +493,7 @@ int avionic_engine_create(const avionic_engine_config *cfg, avionic_engine **eng
       // default: 90% of the device memory free now
       size_t free_b = 0, total_b = 0;
       AV_HIP(hipMemGetInfo(&free_b, &total_b));
-      e->cfg.hbm_budget_bytes = free_b / 10 * 9;
+      e->cfg.hbm_budget_bytes = (free_b + pooled_bytes()) / 10 * 9;
     }
     AV_HIP(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     AV_HIP(hipStreamCreateWithFlags(&e->copy_stream, hipStreamNonBlocking));
@@ -507,6 +513,7 @@ int avionic_engine_destroy(avionic_engine *engine) {
   return eguard([&] {
     if (!engine) return;
     (void)hipStreamSynchronize(engine->stream);
+    (void)hipStreamSynchronize(engine->side);
     delete engine;
   });
 }
@@ -577,28 +584,36 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
     AV_HIP(hipEventRecord(e->ev_req, (hipStream_t)d->stream));
     AV_HIP(hipStreamWaitEvent(st, e->ev_req, 0));
     const long N = s->N, K = std::max(1L, s->K);
-    s->x.ensure(sizeof(float2) * P * N);
-    s->ext.ensure(sizeof(float2) * P * N);
-    s->y.ensure(dual_bytes(s->ds) * D * N);
-    s->z.ensure(sizeof(float2) * K);
-    s->d.ensure(sizeof(float2) * K);
-    s->kcol.ensure(sizeof(float2) * K);
-    s->zhat.ensure(sizeof(float2) * K);
-    s->khz.ensure(sizeof(float2) * N);
-    s->b1.ensure(sizeof(float2) * (size_t)s->C * s->H * s->W);
-    s->slog.ensure(sizeof(double) * std::max(1, s->maxit));
-    s->tlog.ensure(sizeof(double) * std::max(1, s->maxit));
     const Grid3 g{s->W, s->H, s->T, N};
     const int nvb = step_blocks(g);
     const int nrb = s->cart ? s->cart->plan().row_blocks() : 0;
     const int npk = s->cart ? nrb : s->op->max_partials();
-    s->preg.ensure(sizeof(double) * 2 * nvb);
-    s->pk.ensure(sizeof(double) * std::max(1, npk));
+    PoolLayout layout;
+    layout.add(s->x, sizeof(float2) * P * N);
+    layout.add(s->ext, sizeof(float2) * P * N);
+    layout.add(s->y, dual_bytes(s->ds) * D * N);
+    layout.add(s->z, sizeof(float2) * K);
+    layout.add(s->d, sizeof(float2) * K);
+    layout.add(s->kcol, sizeof(float2) * K);
+    layout.add(s->zhat, sizeof(float2) * K);
+    layout.add(s->khz, sizeof(float2) * N);
+    layout.add(s->b1, sizeof(float2) * (size_t)s->C * s->H * s->W);
+    layout.add(s->slog, sizeof(double) * std::max(1, s->maxit));
+    layout.add(s->tlog, sizeof(double) * std::max(1, s->maxit));
+    layout.add(s->preg, sizeof(double) * 2 * nvb);
+    layout.add(s->pk, sizeof(double) * std::max(1, npk));
+    layout.add(s->sc, sizeof(DevScalars));
     if (s->gap_enabled()) {
       const size_t np = gap_partials(g, *s->op);
-      s->gap_a.ensure(sizeof(double) * np);
-      s->gap_b.ensure(sizeof(double) * np);
+      layout.add(s->gap_a, sizeof(double) * np);
+      layout.add(s->gap_b, sizeof(double) * np);
     }
+    s->mem = PoolBlock(layout.total);
+    layout.cut(s->mem);
+    s->busy = st;
+    // kept blocks stay within the engine's budget beside the held requests
+    const size_t held = e->used + s->bytes;
+    trim_pool(e->cfg.hbm_budget_bytes > held ? e->cfg.hbm_budget_bytes - held : 0);
     AV_HIP(hipMemsetAsync(s->x.p, 0, s->x.bytes, st));
     AV_HIP(hipMemsetAsync(s->y.p, 0, s->y.bytes, st));
     AV_HIP(hipMemsetAsync(s->z.p, 0, s->z.bytes, st));
@@ -627,9 +642,9 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
     hs.iter = 0;
     hs.maxit = s->maxit;
     hs.schedule = s->params.adaptSchedule;
-    s->sc.ensure(sizeof(DevScalars));
     AV_HIP(hipMemcpyAsync(s->sc.p, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
     AV_HIP(hipStreamSynchronize(st));  // the caller may release its inputs now
+    s->busy = nullptr;
 
     const double d6[6] = {s->params.dx, s->params.dy, s->params.dt,
                           s->params.dx2, s->params.dy2, s->params.dt2};
@@ -737,6 +752,7 @@ int avionic_engine_poll(avionic_engine *e, long long id, float *x_out, void *str
     AV_CHECK(x_out != nullptr, "x_out is null");
     hipStream_t us = (hipStream_t)stream;
     AV_HIP(hipStreamSynchronize(e->stream));
+    AV_HIP(hipStreamSynchronize(e->side));  // its buffers go back to the pool below
     DevScalars hs{};
     AV_HIP(hipMemcpy(&hs, s->sc.p, sizeof(hs), hipMemcpyDeviceToHost));
     AV_HIP(hipMemcpyAsync(x_out, s->x.p, sizeof(float2) * s->N, hipMemcpyDeviceToDevice, us));
@@ -765,6 +781,7 @@ int avionic_engine_cancel(avionic_engine *e, long long id) {
     if (it == e->slots.end()) throw Error(AVIONIC_E_NOTFOUND, "unknown request id");
     Slot *s = it->second.get();
     AV_HIP(hipStreamSynchronize(e->stream));
+    AV_HIP(hipStreamSynchronize(e->side));
     for (auto &kv : e->groups) {
       auto &v = kv.second.slots;
       auto f = std::find(v.begin(), v.end(), s);

@@ -2,6 +2,7 @@
 // operator's column and row passes are in k_cart_col.hip and k_cart_row.hip.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "cart_device.hpp"
@@ -155,7 +156,7 @@ static void pick_stages(int m, int most, double cost, int n, int *r, double &bes
     }
 }
 
-void make_fft_plan(int L, FftPlan &p, void **d_tw) {
+void fft_plan_host(int L, FftPlan &p, std::vector<float2> &tw) {
   AV_CHECK(L >= 1 && L <= kMaxFftLen, "FFT length out of range (1..1024)");
   p = FftPlan{};
   p.L = L;
@@ -177,20 +178,51 @@ void make_fft_plan(int L, FftPlan &p, void **d_tw) {
   double best = 1e30;
   pick_stages(L, kMaxRadix, 0.0, 0, r, best, p);
   while (p.nx < 2) p.rx[p.nx++] = 1;
-  std::vector<float2> tw(L);
+  tw.resize(L);
   for (int k = 0; k < L; ++k) {
     const double a = -2.0 * M_PI * (double)k / (double)L;
     tw[k] = make_float2((float)std::cos(a), (float)std::sin(a));
   }
+}
+
+void make_fft_plan(int L, FftPlan &p, void **d_tw) {
+  std::vector<float2> tw;
+  fft_plan_host(L, p, tw);
   AV_HIP(hipMalloc(d_tw, sizeof(float2) * L));
   AV_HIP(hipMemcpy(*d_tw, tw.data(), sizeof(float2) * L, hipMemcpyHostToDevice));
   AV_HIP(hipStreamSynchronize(nullptr));  // landed before any stream reads it
   p.tw = (const float2 *)*d_tw;
 }
 
+// One block per mask row (t, y): its sum of squares, or -1 when no value is
+// nonzero (a NaN counts as nonzero).
+__global__ __launch_bounds__(NT) void k_mask_rows(const float *__restrict__ mask, int W,
+                                                  double *__restrict__ out) {
+  __shared__ double red[NT];
+  __shared__ int any;
+  if (threadIdx.x == 0) any = 0;
+  __syncthreads();
+  double acc = 0.0;
+  int mine = 0;
+  for (int x = threadIdx.x; x < W; x += NT) {
+    const float v = mask[(long)blockIdx.x * W + x];
+    acc += (double)v * v;
+    mine |= v != 0.f;
+  }
+  if (mine) any = 1;
+  const double s = block_sum(acc, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = any ? s : -1.0;
+}
+// Mask values of the sampled rows (ones without a mask), one block per row.
+__global__ void k_mask_gather(const float *__restrict__ mask, const int *__restrict__ src, int W,
+                              float *__restrict__ mrows) {
+  const long r = blockIdx.x;
+  for (int x = threadIdx.x; x < W; x += blockDim.x)
+    mrows[r * W + x] = mask ? mask[(long)src[r] * W + x] : 1.f;
+}
+
 CartPlan::~CartPlan() {
-  for (void *p : {d_row_off, d_rows, d_mrows, d_rowinfo, d_rowmap, d_twx, d_twy})
-    if (p) (void)hipFree(p);
+  if (d_tables) (void)hipFree(d_tables);
 }
 
 void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered, hipStream_t s) {
@@ -200,31 +232,30 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   g.W = W; g.H = H; g.C = C; g.T = T;
   g.centered = centered ? 1 : 0;
   g.scale = (float)(1.0 / std::sqrt((double)H * W));
-  const long HW = (long)H * W;
-  std::vector<float> hm;
   has_mask = mask != nullptr;
+  std::vector<double> sums((size_t)T * H, 0.0);  // -1: row not sampled
   if (mask) {
-    hm.resize((size_t)HW * T);
-    AV_HIP(hipMemcpyAsync(hm.data(), mask, sizeof(float) * hm.size(), hipMemcpyDeviceToHost, s));
-    AV_HIP(hipStreamSynchronize(s));
+    double *d = nullptr;
+    AV_HIP(hipMalloc((void **)&d, sizeof(double) * sums.size()));
+    hipLaunchKernelGGL(k_mask_rows, dim3((unsigned)sums.size()), dim3(NT), 0, s, mask, W, d);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(sums.data(), d, sizeof(double) * sums.size(), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    (void)hipFree(d);
+    AV_HIP(e);
   }
   h_row_off.assign(T + 1, 0);
   h_rows.clear();
-  std::vector<float> mrows;
+  std::vector<int> src;  // mask row t H + y of each sampled row
   mask_norm2 = 0.0;
   for (int t = 0; t < T; ++t) {
     for (int y = 0; y < H; ++y) {
-      bool any = !mask;
-      if (mask)
-        for (int x = 0; x < W; ++x) {
-          const float v = hm[(size_t)t * HW + (size_t)y * W + x];
-          mask_norm2 += (double)v * v;
-          if (v != 0.f) any = true;
-        }
-      if (any) {
-        h_rows.push_back(y);
-        for (int x = 0; x < W; ++x) mrows.push_back(mask ? hm[(size_t)t * HW + (size_t)y * W + x] : 1.f);
-      }
+      const double v = sums[(size_t)t * H + y];
+      if (v == -1.0) continue;
+      mask_norm2 += v;
+      h_rows.push_back(y);
+      src.push_back(t * H + y);
     }
     h_row_off[t + 1] = (int)h_rows.size();
   }
@@ -240,22 +271,40 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
     for (int c = 0; c < C; ++c)
       for (int k = 0; k < S; ++k) info.push_back(make_int4(t, c, r0 + k, h_rows[r0 + k]));
   }
-  auto up = [&](void **dst, const void *src, size_t bytes) {
-    AV_HIP(hipMalloc(dst, bytes > 0 ? bytes : 16));
-    if (bytes) AV_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
+  std::vector<float2> twx, twy;
+  fft_plan_host(W, g.pw, twx);
+  fft_plan_host(H, g.ph, twy);
+  // one allocation and one copy for all tables, then the mask rows behind them
+  std::vector<char> host;
+  auto put = [&](const void *p, size_t bytes) {
+    const size_t at = host.size();
+    host.resize(at + (bytes + 255) / 256 * 256);
+    if (bytes) std::memcpy(host.data() + at, p, bytes);
+    return at;
   };
-  up(&d_row_off, h_row_off.data(), sizeof(int) * h_row_off.size());
-  up(&d_rows, h_rows.data(), sizeof(int) * h_rows.size());
-  up(&d_mrows, mrows.data(), sizeof(float) * mrows.size());
-  up(&d_rowinfo, info.data(), sizeof(int4) * info.size());
-  up(&d_rowmap, rowmap.data(), sizeof(int) * rowmap.size());
-  g.row_off = (const int *)d_row_off;
-  g.rows = (const int *)d_rows;
-  g.mrows = (const float *)d_mrows;
-  g.rowinfo = (const int4 *)d_rowinfo;
-  g.rowmap = (const int *)d_rowmap;
-  make_fft_plan(W, g.pw, &d_twx);
-  make_fft_plan(H, g.ph, &d_twy);
+  const size_t o_off = put(h_row_off.data(), sizeof(int) * h_row_off.size());
+  const size_t o_rows = put(h_rows.data(), sizeof(int) * h_rows.size());
+  const size_t o_src = put(src.data(), sizeof(int) * src.size());
+  const size_t o_info = put(info.data(), sizeof(int4) * info.size());
+  const size_t o_map = put(rowmap.data(), sizeof(int) * rowmap.size());
+  const size_t o_twx = put(twx.data(), sizeof(float2) * twx.size());
+  const size_t o_twy = put(twy.data(), sizeof(float2) * twy.size());
+  const size_t o_mrows = host.size();
+  AV_HIP(hipMalloc(&d_tables, o_mrows + sizeof(float) * (size_t)g.nrows * W + 256));
+  char *base = (char *)d_tables;
+  AV_HIP(hipMemcpy(base, host.data(), host.size(), hipMemcpyHostToDevice));
+  g.row_off = (const int *)(base + o_off);
+  g.rows = (const int *)(base + o_rows);
+  g.rowinfo = (const int4 *)(base + o_info);
+  g.rowmap = (const int *)(base + o_map);
+  g.mrows = (const float *)(base + o_mrows);
+  g.pw.tw = (const float2 *)(base + o_twx);
+  g.ph.tw = (const float2 *)(base + o_twy);
+  if (g.nrows > 0) {
+    hipLaunchKernelGGL(k_mask_gather, dim3((unsigned)g.nrows), dim3(NT), 0, nullptr, mask,
+                       (const int *)(base + o_src), W, (float *)(base + o_mrows));
+    AV_LAUNCH_CHECK();
+  }
   set_col_tiles(g, wide_col_blocks(g) >= kColWideBlocks);
   if (g.pw.ra) {
     g.ljb = log2_ceil(g.pw.ra);
@@ -266,10 +315,10 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   }
   g.wide_col = plan_is_wide(g.ph) ? 1 : 0;
   g.wide_row = plan_is_wide(g.pw) ? 1 : 0;
-  // The tables above come from pageable host memory: such a copy (on the
-  // null stream) may return before its data has landed, and the kernels that
-  // index with them may run on non-blocking streams, which do not wait for
-  // the null stream.  Waiting for the null stream alone leaves those streams'
+  // The tables above come from pageable host memory (such a copy, on the null
+  // stream, may return before its data has landed) and from a kernel there, and
+  // the kernels that index with them may run on non-blocking streams, which do
+  // not wait for the null stream.  Waiting for the null stream alone leaves those streams'
   // own work running.
   AV_HIP(hipStreamSynchronize(nullptr));
 }

@@ -1,0 +1,128 @@
+#include "pool.hpp"
+
+#include <hip/hip_runtime.h>
+
+#include <deque>
+#include <mutex>
+#include <string>
+
+#include "common.hpp"
+
+namespace avionic {
+
+namespace {
+
+struct Kept {
+  void *p;
+  size_t bytes;
+  int dev;
+};
+struct Pool {
+  std::mutex mu;
+  std::deque<Kept> kept;  // oldest first
+  size_t bytes = 0;
+  int users = 0;
+};
+// Never destroyed: blocks may be given back after static destruction began.
+Pool &pool() {
+  static Pool *p = new Pool;
+  return *p;
+}
+void trim_locked(Pool &g, size_t most) {
+  while (g.bytes > most) {
+    const Kept k = g.kept.front();
+    g.kept.pop_front();
+    g.bytes -= k.bytes;
+    (void)hipFree(k.p);
+  }
+}
+
+}  // namespace
+
+void trim_pool(size_t most) {
+  Pool &g = pool();
+  std::lock_guard<std::mutex> lock(g.mu);
+  trim_locked(g, most);
+}
+
+size_t pooled_bytes() {
+  Pool &g = pool();
+  std::lock_guard<std::mutex> lock(g.mu);
+  return g.bytes;
+}
+
+void *device_alloc(size_t bytes) {
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    trim_pool(0);
+    e = hipMalloc(&p, bytes);
+  }
+  if (e != hipSuccess)
+    throw Error(-2, std::string("hipMalloc(&p, ") + std::to_string(bytes) + "): " + hipGetErrorString(e));
+  return p;
+}
+
+PoolBlock::PoolBlock(size_t need) {
+  AV_HIP(hipGetDevice(&dev));
+  need = need > 0 ? need : 256;
+  {
+    // the smallest kept block that wastes at most half of the size asked for
+    Pool &g = pool();
+    std::lock_guard<std::mutex> lock(g.mu);
+    auto best = g.kept.end();
+    for (auto it = g.kept.begin(); it != g.kept.end(); ++it)
+      if (it->dev == dev && it->bytes >= need && it->bytes - need <= need / 2 &&
+          (best == g.kept.end() || it->bytes < best->bytes))
+        best = it;
+    if (best != g.kept.end()) {
+      p = best->p;
+      bytes = best->bytes;
+      g.bytes -= bytes;
+      g.kept.erase(best);
+      return;
+    }
+  }
+  p = device_alloc(need);
+  bytes = need;
+}
+
+PoolBlock::PoolBlock(PoolBlock &&o) noexcept : p(o.p), bytes(o.bytes), dev(o.dev) { o.p = nullptr; }
+PoolBlock &PoolBlock::operator=(PoolBlock &&o) noexcept {
+  if (this != &o) {
+    give();
+    p = o.p;
+    bytes = o.bytes;
+    dev = o.dev;
+    o.p = nullptr;
+  }
+  return *this;
+}
+
+void PoolBlock::give() {
+  if (!p) return;
+  Pool &g = pool();
+  std::lock_guard<std::mutex> lock(g.mu);
+  if (g.users == 0 || bytes > kPoolBytes) {
+    (void)hipFree(p);
+  } else {
+    trim_locked(g, kPoolBytes - bytes);
+    g.kept.push_back(Kept{p, bytes, dev});
+    g.bytes += bytes;
+  }
+  p = nullptr;
+}
+
+PoolUser::PoolUser() {
+  Pool &g = pool();
+  std::lock_guard<std::mutex> lock(g.mu);
+  ++g.users;
+}
+PoolUser::~PoolUser() {
+  Pool &g = pool();
+  std::lock_guard<std::mutex> lock(g.mu);
+  if (--g.users == 0) trim_locked(g, 0);
+}
+
+}  // namespace avionic

@@ -1,0 +1,74 @@
+// Device memory kept between reconstructions.
+//
+// A reconstruction needs one block of device memory for its state; hipMalloc and
+// hipFree of a dozen buffers cost more than a hundred small iterations (and
+// hipFree waits for the device).  Blocks that are given back are kept, at most
+// kPoolBytes per process, and handed to the next request of a like size on the
+// same device.  They go back to the device when the last solver or engine is
+// destroyed, when the bound is passed (oldest first), and when an allocation
+// fails.  Thread-safe; whoever gives a block back has waited for the streams
+// that use it.
+#pragma once
+
+#include <cstddef>
+
+namespace avionic {
+
+constexpr size_t kPoolBytes = size_t(4) << 30;
+
+// A block of the pool, or none.  Move-only; give() or the destructor returns it.
+class PoolBlock {
+ public:
+  PoolBlock() = default;
+  explicit PoolBlock(size_t bytes);  // throws when the device has no such memory
+  PoolBlock(PoolBlock &&o) noexcept;
+  PoolBlock &operator=(PoolBlock &&o) noexcept;
+  ~PoolBlock() { give(); }
+  void give();
+  void *p = nullptr;
+  size_t bytes = 0;  // at least the size asked for
+  int dev = 0;
+};
+
+// hipMalloc that empties the pool and tries again when memory runs out.
+void *device_alloc(size_t bytes);
+
+// Owners of blocks: the pool is emptied when the last one ends.
+struct PoolUser {
+  PoolUser();
+  ~PoolUser();
+  PoolUser(const PoolUser &) = delete;
+  PoolUser &operator=(const PoolUser &) = delete;
+};
+size_t pooled_bytes();
+// Frees kept blocks, oldest first, until at most `most` bytes are kept.
+void trim_pool(size_t most);
+
+// Part of a block.
+struct DevView {
+  void *p = nullptr;
+  size_t bytes = 0;
+  template <typename T>
+  T *as() const { return (T *)p; }
+};
+// Sizes collected first, then one block cut into 256-byte aligned parts.
+struct PoolLayout {
+  static constexpr int kMost = 20;
+  DevView *view[kMost];
+  int n = 0;
+  size_t total = 0;
+  void add(DevView &v, size_t bytes) {
+    v.bytes = bytes;
+    view[n++] = &v;
+    total += (bytes + 255) / 256 * 256;
+  }
+  void cut(const PoolBlock &b) {
+    char *p = (char *)b.p;
+    for (int i = 0; i < n; ++i) {
+      view[i]->p = p;
+      p += (view[i]->bytes + 255) / 256 * 256;
+    }
+  }
+};
+
+}  // namespace avionic

@@ -379,16 +379,24 @@ void Recon::run(const float2 *data, float2 *xio, const float2 *b1, hipStream_t s
   const int P = primal_components(method), D = dual_components(method);
   const int dstore = params.dualStorage;
   const long K = op->compact_elems();
-  DevBuf x, ext, y, z, d, khz, slog, tlog;
-  x.ensure(sizeof(float2) * (size_t)P * N);
-  ext.ensure(sizeof(float2) * (size_t)P * N);
-  y.ensure(dual_bytes(dstore) * (size_t)D * N);
-  z.ensure(sizeof(float2) * (size_t)std::max(1L, K));
-  d.ensure(sizeof(float2) * (size_t)std::max(1L, K));
-  khz.ensure(sizeof(float2) * (size_t)N);
   const unsigned maxIt = params.maxIt;
-  slog.ensure(sizeof(double) * std::max(1u, maxIt));
-  tlog.ensure(sizeof(double) * std::max(1u, maxIt));
+  DevView x, ext, y, z, d, khz, slog, tlog;
+  PoolLayout layout;
+  layout.add(x, sizeof(float2) * (size_t)P * N);
+  layout.add(ext, sizeof(float2) * (size_t)P * N);
+  layout.add(y, dual_bytes(dstore) * (size_t)D * N);
+  layout.add(z, sizeof(float2) * (size_t)std::max(1L, K));
+  layout.add(d, sizeof(float2) * (size_t)std::max(1L, K));
+  layout.add(khz, sizeof(float2) * (size_t)N);
+  layout.add(slog, sizeof(double) * std::max(1u, maxIt));
+  layout.add(tlog, sizeof(double) * std::max(1u, maxIt));
+  // given back when the run ends, also by an exception: its stream is waited for
+  struct Work {
+    PoolBlock block;
+    hipStream_t s;
+    ~Work() { (void)hipStreamSynchronize(s); }
+  } work{PoolBlock(layout.total), s};
+  layout.cut(work.block);
 
   AV_HIP(hipMemsetAsync(x.p, 0, x.bytes, s));
   AV_HIP(hipMemsetAsync(y.p, 0, y.bytes, s));

@@ -13,6 +13,7 @@
 #include "cartesian.hpp"
 #include "common.hpp"
 #include "opnorm.hpp"
+#include "pool.hpp"
 #include "reg.hpp"
 
 namespace avionic {
@@ -33,7 +34,7 @@ struct DevBuf {
   void ensure(size_t b) {
     if (b <= bytes && p) return;
     release();
-    AV_HIP(hipMalloc(&p, b > 0 ? b : 16));
+    p = device_alloc(b > 0 ? b : 16);
     bytes = b;
   }
   template <typename T>
@@ -177,6 +178,7 @@ class Recon {
   void d6(double out[6]) const;
   void ensure_partials();
   double reduce_pair(const double *partial, int n, int which, hipStream_t s);
+  PoolUser pool_user_;
   DevBuf part_a_, part_b_, scal_;
 };
 
