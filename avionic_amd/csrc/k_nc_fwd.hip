@@ -146,8 +146,9 @@ __global__ __launch_bounds__(NCR) void k_nc_row_fwd(NcGeom g, const float2 *__re
   const int e0 = rp[gy0], e1 = rp[gy0 + nr];
   float2 *pp = part + ((long)t * g.C + cz) * g.M * kNcTaps;  // coil cz + q: M kNcTaps further
   for (int e = e0 + tid; e < e1; e += NCR) {
-    // (partial index m*4 + dy, grid row, first grid column, row weight) and
-    // the column weights: no load here depends on another
+    // (partial index dy M + m, grid row, first grid column, row weight) and the
+    // column weights: no load here depends on another.  Consecutive points of a
+    // spoke stay consecutive in a plane of partials.
     const int4 h = g.rhdr[e];
     const float4 wx = g.rwx[e];
     const int qx = h.z;
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(NCR) void k_nc_row_fwd(NcGeom g, const float2 *__re
       float2 acc = cscale(row[qx], wx.x);
       acc = cadd(acc, cscale(row[wrap_up(qx + 1, Gx)], wx.y));
       acc = cadd(acc, cscale(row[wrap_up(qx + 2, Gx)], wx.z));
-      acc = cadd(acc, cscale(row[wrap_up(qx + 3, Gx)], wx.w));
+      if (wx.w != 0.f) acc = cadd(acc, cscale(row[wrap_up(qx + 3, Gx)], wx.w));  // rare
       pp[(long)q * g.M * kNcTaps + (unsigned)h.x] = cscale(acc, __int_as_float(h.w));
     }
   }
@@ -184,7 +185,6 @@ __global__ __launch_bounds__(NCR) void k_nc_samples(NcGeom g, const float2 *__re
                                                     double *__restrict__ partial) {
   __shared__ double red[NCR];
   const long n = (long)g.T * g.C * g.M;
-  const long CM = (long)g.C * g.M;
   float sigma = 0.f, inv = 0.f;
   if (MODE == kNcDualUpdate) {
     sigma = (float)sc->sigma;
@@ -192,12 +192,13 @@ __global__ __launch_bounds__(NCR) void k_nc_samples(NcGeom g, const float2 *__re
   }
   double acc = 0.0;
   for (long e = (long)blockIdx.x * NCR + threadIdx.x; e < n; e += (long)gridDim.x * NCR) {
-    const long t = e / CM;
-    const long m = e % g.M;
-    const float4 *p4 = reinterpret_cast<const float4 *>(part + e * kNcTaps);
-    const float4 a = p4[0], b = p4[1];
-    float2 v = make_float2(a.x + a.z + b.x + b.z, a.y + a.w + b.y + b.w);
-    v = cscale(v, g.sw[t * g.M + m]);
+    const long pl = e / g.M, m = e - pl * g.M;  // plane (t, c), point
+    const int t = (int)pl / g.C;
+    const float2 *p = part + pl * g.M * kNcTaps + m;
+    const float2 p0 = p[0], p1 = p[g.M], p2 = p[2L * g.M];
+    float2 v = make_float2(p0.x + p1.x + p2.x, p0.y + p1.y + p2.y);
+    if (g.last[t]) v = cadd(v, p[3L * g.M]);
+    v = cscale(v, g.sw[(long)t * g.M + m]);
     if (MODE == kNcApplyK) {
       out[e] = v;
     } else if (MODE == kNcDualUpdate) {

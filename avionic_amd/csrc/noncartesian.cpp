@@ -191,6 +191,7 @@ class NoncartesianOperator : public Operator {
     std::vector<float4> wx4((size_t)T * M), wy4((size_t)T * M);
     std::vector<int> rptr((size_t)T * (Gy + 1));
     std::vector<int4> rhdr;
+    std::vector<int> last(T, 0);  // frames with a point on kNcTaps rows
     std::vector<float4> rwx;
     std::vector<int> cptr((size_t)T * (G2 + 1));
     std::vector<int2> ce;
@@ -228,19 +229,23 @@ class NoncartesianOperator : public Operator {
         wx4[p] = make_float4(w4x[0], w4x[1], w4x[2], w4x[3]);
         wy4[p] = make_float4(w4y[0], w4y[1], w4y[2], w4y[3]);
       }
-      // row -> (point, tap): every point lists all kNcTaps rows (a zero
-      // weight row still writes its partial, so none is left stale)
+      // row -> (point, tap) over the rows with a weight: a kernel of width 3
+      // covers three rows of a point, four only where one is exactly 1.5 away.
+      // The partials of the others are never written and stay zero.
       std::vector<std::vector<int2>> rows(Gy);
       for (long m = 0; m < M; ++m)
         for (int dy = 0; dy < kNcTaps; ++dy)
-          rows[wrap(qy[m] + dy, Gy)].push_back(make_int2((int)m, dy));
+          if (wyd[m * kNcTaps + dy] != 0.0) {
+            rows[wrap(qy[m] + dy, Gy)].push_back(make_int2((int)m, dy));
+            if (dy == kNcTaps - 1) last[t] = 1;
+          }
       int *rp = &rptr[(size_t)t * (Gy + 1)];
       for (int r = 0; r < Gy; ++r) {
         rp[r] = (int)rhdr.size();
         for (const int2 &md : rows[r]) {
           const size_t pi = (size_t)t * M + md.x;
           const float wyd = (&wy4[pi].x)[md.y];
-          rhdr.push_back(make_int4(md.x * kNcTaps + md.y, r, q0[pi].x, __builtin_bit_cast(int, wyd)));
+          rhdr.push_back(make_int4(md.y * (int)M + md.x, r, q0[pi].x, __builtin_bit_cast(int, wyd)));
           rwx.push_back(wx4[pi]);
         }
       }
@@ -281,6 +286,7 @@ class NoncartesianOperator : public Operator {
     up(rptr_, rptr.data(), sizeof(int) * rptr.size());
     up(rhdr_, rhdr.data(), sizeof(int4) * rhdr.size());
     up(rwx_, rwx.data(), sizeof(float4) * rwx.size());
+    up(last_, last.data(), sizeof(int) * last.size());
     up(cptr_, cptr.data(), sizeof(int) * cptr.size());
     up(ce_, ce.data(), sizeof(int2) * ce.size());
     up(q64_, q0.data(), sizeof(int2) * q0.size());
@@ -315,6 +321,7 @@ class NoncartesianOperator : public Operator {
     g_.rptr = rptr_.as<int>();
     g_.rhdr = rhdr_.as<int4>();
     g_.rwx = rwx_.as<float4>();
+    g_.last = last_.as<int>();
     g_.cptr = cptr_.as<int>();
     g_.ce = ce_.as<int2>();
     {
@@ -350,6 +357,8 @@ class NoncartesianOperator : public Operator {
       g_.tce = tce_.as<int2>();
     }
     scratch();
+    AV_HIP(hipMemset(part_.p, 0, part_.bytes));
+    AV_HIP(hipStreamSynchronize(nullptr));
     const NcTiles tiles = tune_tiles(g_, tmp_.as<float2>(), part_.as<float2>());
     g_.CG = tiles.cg;
     g_.RBa = tiles.rows;
@@ -416,7 +425,7 @@ class NoncartesianOperator : public Operator {
   int spf_, nfe_;
   std::vector<float> traj_h_, dens_h_;
   NcGeom g_{};
-  DevBuf dxi_, dyi_, sw_, rptr_, rhdr_, rwx_, cptr_, ce_, tstart_, tcell_, tce_, twx_, twy_, tmp_,
+  DevBuf dxi_, dyi_, sw_, rptr_, rhdr_, rwx_, last_, cptr_, ce_, tstart_, tcell_, tce_, twx_, twy_, tmp_,
       part_;
   DevBuf q64_, w64_, sw64_, cew64_, dxi64_, dyi64_;  // FP64 tables
 
