@@ -248,9 +248,9 @@ void nc_forward_rt(const NcGeom &g, const float2 *u, const float2 *usub, const f
 void launch_nc_forward_grid(const NcGeom &g, const float2 *u, const float2 *usub,
                             const float2 *b1, float2 *tmp, float2 *part, hipStream_t s) {
   switch (nc_ct_len(g)) {
-    case 384: nc_forward_ct<NcPlan384>(g, u, usub, b1, tmp, part, s); return;
+    case 384: nc_forward_ct<NcFwd384>(g, u, usub, b1, tmp, part, s); return;
     case 512: nc_forward_ct<NcPlan512>(g, u, usub, b1, tmp, part, s); return;
-    case 192: nc_forward_ct<NcPlan192>(g, u, usub, b1, tmp, part, s); return;
+    case 192: nc_forward_ct<NcFwd192>(g, u, usub, b1, tmp, part, s); return;
     case 256: nc_forward_ct<NcPlan256>(g, u, usub, b1, tmp, part, s); return;
     default: break;
   }

@@ -32,10 +32,10 @@ __device__ inline int wrap_up(int v, int G) { return v >= G ? v - G : v; }
 
 // Grid transforms: on the geometry's runtime plans (NcPlanRt), or compiled
 // for a grid length in both directions, with XB grid columns per column-pass
-// block (pick_cols at that length): 384 (a 256 x 256 image at oversampling 1.5; 16, 8, 3), 512 (256 x 256 at
-// 2, the reference's default oversampling; 16, 16, 2), 192 and 256 (128 x 128
-// at 1.5 and 2; 16, 4, 3 and 16, 16).  nc_ct_len picks the compiled kernels;
-// they run their stages with the index arithmetic folded into constants.
+// block (pick_cols at that length): 384 (a 256 x 256 image at oversampling
+// 1.5), 512 (256 x 256 at 2, the reference's default oversampling), 192 and 256
+// (128 x 128 at 1.5 and 2).  nc_ct_len picks the compiled kernels; they run
+// their stages with the index arithmetic folded into constants.
 struct NcPlanRt {
   static constexpr int L = 0, XB = 0;
 };
@@ -45,9 +45,15 @@ struct NcCt : F {
   static constexpr int RL = F::R2 > 1 ? F::R2 : F::R1;  // last radix
 };
 using NcPlan384 = NcCt<FftCt<384, 16, 8, 3>, 8>;
-using NcPlan512 = NcCt<FftCt<512, 16, 16, 2>, 8>;
+using NcPlan512 = NcCt<FftCt<512, 8, 8, 8>, 8>;
 using NcPlan192 = NcCt<FftCt<192, 16, 4, 3>, 16>;
 using NcPlan256 = NcCt<FftCt<256, 16, 16>, 16>;
+// K's passes: radices of about equal size keep their lanes equally busy in every
+// stage; K^H's column pass (512 lanes, its sums between) measured faster with
+// the others above.  K at 256x256x30x12: 324 -> 312 us (osf 1.5, against 16, 8,
+// 3), 424 -> 397 us (osf 2, 8, 8, 8 against 16, 16, 2; K^H 481 -> 459 us).
+using NcFwd384 = NcCt<FftCt<384, 8, 8, 6>, 8>;
+using NcFwd192 = NcCt<FftCt<192, 16, 12>, 16>;
 
 // The compiled grid length that applies (0: none): both grid directions have
 // that length and the tiles have the compiled sizes.
