@@ -205,8 +205,12 @@ void nc_adjoint_rt(const NcGeom &g, const float2 *z, const float2 *b1, float2 *t
                    hipStream_t s) {
   const size_t cps_bytes = sizeof(int) * ((size_t)g.XBa * g.Gy + 1);
   const int nXa = (g.Gx + g.XBa - 1) / g.XBa;
-  hipLaunchKernelGGL((k_nc_col_adj<KIND, NcPlanRt, 1>), dim3(nXa, g.T * g.C), dim3(NCC), cps_bytes,
-                     s, g, z, tmp);
+  // two coils per block where the transform has three stages (K^H 224x224x16x8
+  // at osf 2: 186 -> 178 us); two-stage ones lose more blocks than they save
+  // table loads (160x160x24x10 at osf 1.5: 152 -> 157 us)
+  constexpr int NZ = KIND == kPlanTwo ? 1 : 2;
+  hipLaunchKernelGGL((k_nc_col_adj<KIND, NcPlanRt, NZ>), dim3(nXa, g.T * ((g.C + NZ - 1) / NZ)),
+                     dim3(NCC), cps_bytes, s, g, z, tmp);
   AV_LAUNCH_CHECK();
   hipLaunchKernelGGL((k_nc_row_adj<KIND, NcPlanRt>), dim3((g.H + g.RBa - 1) / g.RBa, g.T), dim3(NCR),
                      0, s, g, (const float2 *)tmp, b1, img);
