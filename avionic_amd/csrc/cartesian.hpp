@@ -88,6 +88,13 @@ struct CartPlan {
 // busy in both stages; narrow ones give more blocks.  The results do not depend
 // on the choice.
 void set_col_tiles(CartGeom &g, bool wide);
+// Rows per block of a two-stage row pass: wide fills the lanes of both stages,
+// narrow gives more blocks (and other partial sums).  One operator's calls take
+// the narrow form below two wide blocks per CU, where the length of the chain
+// counts (TV 128x128x12x8: 8.5 -> 6.5 us); the engine always the wide one (64
+// such requests together: 113 -> 100 us).
+void set_row_tiles(CartGeom &g, bool wide);
+constexpr int kRowWideBlocks = 512;
 // Blocks of a column pass on wide tiles, and the count from which wide tiles
 // are taken: two blocks per CU.
 long wide_col_blocks(const CartGeom &g);

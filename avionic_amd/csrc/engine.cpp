@@ -586,7 +586,12 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
     const long N = s->N, K = std::max(1L, s->K);
     const Grid3 g{s->W, s->H, s->T, N};
     const int nvb = step_blocks(g);
-    const int nrb = s->cart ? s->cart->plan().row_blocks() : 0;
+    Task &t = s->task;
+    if (s->cart) {  // else zero: no column / row blocks
+      t.cg = s->cart->plan().g;
+      set_row_tiles(t.cg, true);
+    }
+    const int nrb = s->cart ? (int)((t.cg.nrows_c + t.cg.RB - 1) / t.cg.RB) : 0;
     const int npk = s->cart ? nrb : s->op->max_partials();
     PoolLayout layout;
     layout.add(s->x, sizeof(float2) * P * N);
@@ -648,10 +653,8 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
 
     const double d6[6] = {s->params.dx, s->params.dy, s->params.dt,
                           s->params.dx2, s->params.dy2, s->params.dt2};
-    Task &t = s->task;
     t.g = g;
     t.rp = make_reg_params(s->method, d6, s->params.alpha0, s->params.alpha1, s->params.alpha);
-    if (s->cart) t.cg = s->cart->plan().g;  // else zero: no column / row blocks
     t.x = s->x.as<float2>();
     t.ext = s->ext.as<float2>();
     t.y = s->y.p;

@@ -117,6 +117,15 @@ void set_col_tiles(CartGeom &g, bool wide) {
   g.lxb = log2_ceil(g.XB);
   g.nxb = (g.W + g.XB - 1) / g.XB;
 }
+void set_row_tiles(CartGeom &g, bool wide) {
+  if (!g.pw.ra) {
+    g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / g.W));
+    return;
+  }
+  g.ljb = log2_ceil(g.pw.ra);
+  g.lja = wide ? std::max(log2_ceil(g.pw.rb), g.ljb - log2_ceil(two_most(g.pw.rb))) : g.ljb;
+  g.RB = NT >> g.lja;
+}
 long wide_col_blocks(const CartGeom &g) {
   const int xb = col_tile(g, true);
   return (long)((g.W + xb - 1) / xb) * g.T;
@@ -306,13 +315,8 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
     AV_LAUNCH_CHECK();
   }
   set_col_tiles(g, wide_col_blocks(g) >= kColWideBlocks);
-  if (g.pw.ra) {
-    g.ljb = log2_ceil(g.pw.ra);
-    g.lja = std::max(log2_ceil(g.pw.rb), g.ljb - log2_ceil(two_most(g.pw.rb)));
-    g.RB = NT >> g.lja;
-  } else {
-    g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / W));
-  }
+  set_row_tiles(g, true);
+  if (row_blocks() < kRowWideBlocks) set_row_tiles(g, false);
   g.wide_col = plan_is_wide(g.ph) ? 1 : 0;
   g.wide_row = plan_is_wide(g.pw) ? 1 : 0;
   // The tables above come from pageable host memory (such a copy, on the null
