@@ -107,9 +107,10 @@ struct Group {
   std::vector<int> cands;          // candidate variants of the launch set
   std::vector<float> samples[kVariants];
   std::array<long, 8> sig{};       // launch-set signature (decision cache key)
-  void drop_graphs(int keep = -1) {
+  // Only after a wait for the stream that they were launched on: an event after
+  // a launch says that its kernels ran, not that the runtime is done with it.
+  void drop_graphs() {
     for (int v = 0; v < kVariants; ++v) {
-      if (v == keep) continue;
       if (g_step[v]) (void)hipGraphExecDestroy(g_step[v]);
       if (g_plain[v]) (void)hipGraphExecDestroy(g_plain[v]);
       g_step[v] = g_plain[v] = nullptr;
@@ -412,8 +413,7 @@ struct avionic_engine {
     g.variant = best;
     g.tuning = false;
     tuned[g.sig] = best;
-    tunings += 1;
-    g.drop_graphs(best);
+    tunings += 1;  // the others' graphs stay until the next rebuild
   }
 };
 

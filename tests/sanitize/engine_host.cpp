@@ -1,0 +1,158 @@
+// Host side of the engine and the solvers over the stand-in HIP runtime
+// (hip_stub.cpp): built with AddressSanitizer and UndefinedBehaviorSanitizer and
+// run by tests/test_host_runtime.py, one scenario per run.  Kernels do nothing
+// there, so no result is checked, only what the host does around them.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "../../include/avionic.h"
+#include "hip_stub.hpp"
+
+#define CHECK(cond)                                                              \
+  do {                                                                           \
+    if (!(cond)) {                                                               \
+      std::fprintf(stderr, "engine_host: line %d: %s\n", __LINE__, #cond);       \
+      std::exit(1);                                                              \
+    }                                                                            \
+  } while (0)
+
+namespace {
+
+constexpr size_t kMiB = size_t(1) << 20;
+
+float *dev(size_t floats) {
+  void *p = nullptr;
+  CHECK(hipMalloc(&p, sizeof(float) * floats) == hipSuccess);
+  for (size_t i = 0; i < floats; ++i) static_cast<float *>(p)[i] = 1.f;
+  return static_cast<float *>(p);
+}
+// A request of a method (AVIONIC_*), its inputs allocated here.
+struct Req {
+  avionic_request_desc d{};
+  avionic_params p{};
+  Req(int method, unsigned T, unsigned H, unsigned W, unsigned C, unsigned its, int dual) {
+    CHECK(avionic_default_params((avionic_method)method, &p) == 0);
+    p.maxIt = its;
+    p.dualStorage = dual;
+    p.adaptLambda = 0;
+    p.lambda = 1.0;
+    if (method == AVIONIC_TVTEMP) p.dt = 0.8;
+    d.method = (avionic_method)method;
+    d.width = W, d.height = H, d.coils = C, d.frames = T;
+    const size_t n = (size_t)T * H * W;
+    mask = dev(n), data = dev(2 * n * C), b1 = dev((size_t)2 * C * H * W), out = dev(2 * n);
+    d.mask = mask, d.data = data, d.b1 = b1;
+  }
+  Req(Req &&o) : d(o.d), p(o.p), mask(o.mask), data(o.data), b1(o.b1), out(o.out) { o.mask = nullptr; }
+  ~Req() {
+    if (!mask) return;
+    for (float *f : {mask, data, b1, out}) (void)hipFree(f);
+  }
+  int submit(avionic_engine *e, long long *id) {
+    d.params = &p;
+    return avionic_engine_submit(e, &d, id);
+  }
+  float *mask, *data, *b1, *out;
+};
+avionic_engine_config config(int graphs, int tick) {
+  avionic_engine_config c{};
+  c.use_graphs = graphs;
+  c.iterations_per_tick = tick;
+  c.max_queue = -1;
+  return c;
+}
+avionic_engine *engine(const avionic_engine_config &c) {
+  avionic_engine *e = nullptr;
+  CHECK(avionic_engine_create(&c, &e) == 0);
+  return e;
+}
+avionic_engine_counts counts(const avionic_engine *e) {
+  avionic_engine_counts c{};
+  CHECK(avionic_engine_counters(e, &c) == 0);
+  return c;
+}
+// Submits every request and steps the engine until each was polled.
+void run_all(avionic_engine *e, std::vector<Req> &reqs) {
+  std::vector<long long> id(reqs.size());
+  for (size_t i = 0; i < reqs.size(); ++i) CHECK(reqs[i].submit(e, &id[i]) == 0);
+  size_t left = reqs.size();
+  for (int steps = 0; left > 0; ++steps) {
+    CHECK(steps < 10000 && avionic_engine_step(e, nullptr) >= 0);
+    for (size_t i = 0; i < reqs.size(); ++i)
+      if (id[i] >= 0) {
+        const int r = avionic_engine_poll(e, id[i], reqs[i].out, nullptr);
+        CHECK(r >= 0);
+        if (r == 1) id[i] = -1, --left;
+      }
+  }
+}
+
+// Requests of every method and plan kind in one engine, with a cancel, in-loop
+// gaps and a cap on the running ones; the step log of an unfinished request.
+void mixed() {
+  for (int graphs : {1, 0}) {
+    avionic_engine_config c = config(graphs, 3);
+    c.max_batch = 4;
+    avionic_engine *e = engine(c);
+    std::vector<Req> r;
+    r.emplace_back(2, 4, 32, 32, 4, 60, 0);
+    r.emplace_back(0, 3, 24, 40, 3, 45, 0);
+    r.emplace_back(1, 5, 16, 16, 2, 70, 0);
+    r.emplace_back(2, 3, 20, 28, 3, 30, 1);
+    r.emplace_back(3, 4, 24, 24, 3, 50, 0);
+    r.emplace_back(4, 3, 24, 32, 2, 50, 2);
+    r.emplace_back(1, 3, 39, 55, 3, 50, 2);
+    r.emplace_back(0, 2, 300, 250, 2, 30, 0);
+    r[2].d.debug = 1;
+    r[2].d.debugstep = 7;
+    r[0].p.stopPDGap = 1e-9;
+    Req gone(2, 2, 32, 32, 5, 55, 0);
+    long long id = 0;
+    CHECK(gone.submit(e, &id) == 0);
+    CHECK(avionic_engine_step(e, nullptr) >= 0);
+    double sig[64], tau[64];
+    size_t n = 64;
+    CHECK(avionic_engine_get_step_log(e, id, sig, tau, &n) == 0 && n == 3);
+    CHECK(avionic_engine_cancel(e, id) == 0);
+    run_all(e, r);
+    CHECK(counts(e).held == 0 && counts(e).bytes_held == 0);
+    CHECK(avionic_engine_destroy(e) == 0);
+  }
+}
+
+// A launch set whose variants are timed while its iterations are replayed from
+// graphs: the executables of the variants that lose are destroyed only once
+// their stream has been waited for.
+void variants() {
+  for (int tick : {1, 13}) {
+    avionic_engine *e = engine(config(1, tick));
+    std::vector<Req> r;
+    r.emplace_back(2, 4, 32, 48, 3, 120, 2);
+    r.emplace_back(2, 4, 32, 48, 3, 120, 2);
+    run_all(e, r);
+    CHECK(counts(e).launch_tunings == 1);
+    run_all(e, r);  // the same launch set: the decision is reused
+    CHECK(counts(e).launch_tunings == 1);
+    CHECK(avionic_engine_destroy(e) == 0);
+  }
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  stub_set_memory(4096 * kMiB);
+  if (what == "mixed") mixed();
+  else if (what == "variants") variants();
+  else CHECK(!"a scenario");
+  CHECK(stub_launches() > 0);
+  CHECK(stub_faults() == 0);
+  CHECK(stub_memory_held() == 0);
+  std::printf("engine_host: %s ok\n", what.c_str());
+  return 0;
+}
