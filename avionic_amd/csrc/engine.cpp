@@ -93,6 +93,30 @@ inline int variant_of(int lanes, bool col_first) { return (lanes == 1 ? 2 : 0) +
 // iterations unchanged, over this many plain iterations per candidate.
 constexpr int kTuneAfter = 8, kTuneSamples = 3;
 
+// A stream capture and its graph; an exception on the way ends the capture, so
+// that the engine's streams can be used again.
+struct Capture {
+  hipStream_t stream;
+  hipGraph_t graph = nullptr;
+  bool open = true;
+  explicit Capture(hipStream_t s) : stream(s) {
+    AV_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+  }
+  Capture(const Capture &) = delete;
+  Capture &operator=(const Capture &) = delete;
+  void end() {
+    open = false;
+    AV_HIP(hipStreamEndCapture(stream, &graph));
+  }
+  ~Capture() {
+    if (open) {
+      (void)hipStreamEndCapture(stream, &graph);
+      (void)hipGetLastError();
+    }
+    if (graph) (void)hipGraphDestroy(graph);
+  }
+};
+
 struct Group {
   int method = 0;
   int ds = 0;  // dual storage
@@ -378,12 +402,10 @@ struct avionic_engine {
       if (!ex) {
         TraceRange tr("avionic_engine_capture");
         const auto t0 = std::chrono::steady_clock::now();
-        hipGraph_t graph = nullptr;
-        AV_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        Capture cap(stream);
         launch_iteration(g.method, g.ds, g.table.as<Task>(), n, gr, with_step, st, hooks);
-        AV_HIP(hipStreamEndCapture(stream, &graph));
-        AV_HIP(hipGraphInstantiate(&ex, graph, nullptr, nullptr, 0));
-        (void)hipGraphDestroy(graph);
+        cap.end();
+        AV_HIP(hipGraphInstantiate(&ex, cap.graph, nullptr, nullptr, 0));
         captures += 1;
         capture_ms +=
             std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -142,6 +142,29 @@ void variants() {
   }
 }
 
+// A launch that fails anywhere in the first iterations, their captures among
+// them: the step reports it, no stream is left in a capture, and the engine goes
+// on.
+void capture_error() {
+  avionic_engine *e = engine(config(1, 1));
+  for (long n = 1; n <= 30; ++n) {
+    Req r(1, 3, 24, 32, 2, 15, 0);
+    long long id = 0;
+    CHECK(r.submit(e, &id) == 0);
+    stub_fail_launch(n);
+    int rc = 0, steps = 0;
+    do rc = avionic_engine_step(e, nullptr);
+    while (rc >= 0 && ++steps < 13);
+    CHECK(rc < 0);
+    CHECK(avionic_engine_cancel(e, id) == 0);
+    std::vector<Req> again;
+    again.emplace_back(1, 3, 24, 32, 2, 15, 0);
+    run_all(e, again);
+    CHECK(stub_graphs() == 0);
+  }
+  CHECK(avionic_engine_destroy(e) == 0);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -149,6 +172,7 @@ int main(int argc, char **argv) {
   stub_set_memory(4096 * kMiB);
   if (what == "mixed") mixed();
   else if (what == "variants") variants();
+  else if (what == "capture_error") capture_error();
   else CHECK(!"a scenario");
   CHECK(stub_launches() > 0);
   CHECK(stub_faults() == 0);

@@ -51,7 +51,7 @@ std::set<void *> execs;
 std::map<void *, size_t> device;
 size_t cap = size_t(1) << 40, held = 0, peak = 0;
 int faults = 0;
-long launches = 0;
+long launches = 0, graphs = 0, fail_in = 0;
 double clock_ms = 0.0;
 Graph *building = nullptr;
 std::thread::id builder;       // the thread that captures (thread-local mode)
@@ -117,6 +117,8 @@ size_t stub_memory_held() { return held; }
 size_t stub_memory_peak() { return peak; }
 void stub_reset_peak() { peak = held; }
 long stub_launches() { return launches; }
+long stub_graphs() { return graphs; }
+void stub_fail_launch(long n) { fail_in = n; }
 
 extern "C" {
 
@@ -271,6 +273,7 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   Stream *p = of(s);
   if (building || s == nullptr) fault("capture begun inside another, or on the null stream");
   building = new Graph;
+  ++graphs;
   builder = std::this_thread::get_id();
   p->capturing = p->origin = true;
   joined.clear();
@@ -286,19 +289,20 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
   for (Stream *j : joined) j->capturing = false;
   joined.clear();
   p->capturing = p->origin = false;
-  if (building->nodes == 0) fault("empty capture");
   *g = reinterpret_cast<hipGraph_t>(building);
   building = nullptr;
   return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
   std::lock_guard<std::recursive_mutex> l(mu);
+  if (fail_in > 0 && --fail_in == 0) return hipErrorInvalidValue;
   Exec *p = new Exec;
   execs.insert(p);
   *e = reinterpret_cast<hipGraphExec_t>(p);
   return hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t g) {
+  --graphs;
   delete reinterpret_cast<Graph *>(g);
   return hipSuccess;
 }
@@ -365,6 +369,7 @@ hipError_t hipLaunchKernel(const void *, dim3 g, dim3 b, void **, size_t shared,
   if (!b.x || b.x * b.y * b.z > 1024) fault("launch block out of range");
   if (shared > 160 * 1024) fault("launch with more LDS than a CU has");
   ++launches;
+  if (fail_in > 0 && --fail_in == 0) return fail(hipErrorInvalidValue);
   put(of(s), [] {});
   return hipSuccess;
 }
