@@ -147,7 +147,8 @@ void variants() {
 // on.
 void capture_error() {
   avionic_engine *e = engine(config(1, 1));
-  for (long n = 1; n <= 30; ++n) {
+  long n = 1;
+  for (bool failed = true; failed; ++n) {
     Req r(1, 3, 24, 32, 2, 15, 0);
     long long id = 0;
     CHECK(r.submit(e, &id) == 0);
@@ -155,13 +156,15 @@ void capture_error() {
     int rc = 0, steps = 0;
     do rc = avionic_engine_step(e, nullptr);
     while (rc >= 0 && ++steps < 13);
-    CHECK(rc < 0);
+    stub_fail_launch(0);
+    failed = rc < 0;
     CHECK(avionic_engine_cancel(e, id) == 0);
     std::vector<Req> again;
     again.emplace_back(1, 3, 24, 32, 2, 15, 0);
     run_all(e, again);
     CHECK(stub_graphs() == 0);
   }
+  CHECK(n > 15);  // the launches and instantiations of two iteration graphs
   CHECK(avionic_engine_destroy(e) == 0);
 }
 
