@@ -669,17 +669,17 @@ class Engine:
     which submit returns None (default 0: no queue; < 0: unbounded).
     voxels_per_lane: 1 runs the dual / primal updates with one voxel per lane;
     0 (default) with a pair of voxels per lane for requests of even width.
-    fixed_launch: keep the default launch variant; by default a launch set
-    that has run 8 plain iterations unchanged times its variants (one voxel
-    or a pair per lane, column pass before or after the dual update; all give
-    the same bits) and keeps the fastest."""
+    fixed_launch: -1 lets a launch set that has run 8 plain iterations unchanged
+    time its variants (one voxel or a pair per lane, column pass before or after
+    the dual update; all give the same bits) and keep the fastest; otherwise
+    every launch set runs the default variant."""
 
     def __init__(self, hbm_budget_bytes=0, use_graphs=True, max_batch=0, iterations_per_tick=1,
                  resident_bytes_cap=0, max_queue=0, voxels_per_lane=0, fixed_launch=False):
         L = _engine_lib()
         cfg = _EngineConfig(int(hbm_budget_bytes), int(bool(use_graphs)), int(max_batch),
                             int(iterations_per_tick), int(resident_bytes_cap), int(max_queue),
-                            int(voxels_per_lane), int(bool(fixed_launch)))
+                            int(voxels_per_lane), int(fixed_launch))
         h = ctypes.c_void_p()
         _check(L.avionic_engine_create(ctypes.byref(cfg), ctypes.byref(h)))
         self._h = h

@@ -226,7 +226,7 @@ def small_leg(A, synth, torch, dev, B, steps, warmup):
     c64 = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.complex64)).to(dev)
     data, b1, x0 = c64(inp["data"]), c64(inp["b1"]), c64(inp["x0"])
     mask = torch.from_numpy(np.ascontiguousarray(inp["mask"], np.float32)).to(dev)
-    untimed = STEP_RULE_PHASE + TUNE_PHASE + warmup
+    untimed = STEP_RULE_PHASE + SETTLE_PHASE + warmup
     params = dict(wl.params, maxIt=untimed + steps + 10, adaptLambda=0)
 
     def run(use_graphs, n):
@@ -254,10 +254,7 @@ FIXTURE_ITERATIONS = {"tv_128x12x8": 500, "tgv2_256x25x12": 1000, "ictgv2_256x30
 LAMBDA_KD = {"tv": (0.4 * 0.2991, 10.0 * 0.2991), "tgv2": (0.4 * 0.2991, 10.0 * 0.2991),
              "ictgv2": (0.4 / (5.1191 * 0.35), 10.0 / (5.1191 * 0.35))}
 STEP_RULE_PHASE = 10  # iterations k < 10 adapt sigma / tau every iteration
-# The engine times its launch variants once a launch set has run 8 plain
-# iterations unchanged, over 3 plain iterations per variant (at most 4): 20
-# more untimed iterations keep that out of the timed region.
-TUNE_PHASE = 20
+SETTLE_PHASE = 20  # plain iterations more before the warmup (graphs captured, clocks up)
 
 
 def input_digest(data, b1, x0, mask):
@@ -316,7 +313,7 @@ def cartesian_leg(A, synth, torch, dev, name, batch, dual, steps, warmup, plain=
                                                                    inp["x0"], inp["mask"]))
     if fixture_ok:
         lam = fx["lam"]
-    run_its = STEP_RULE_PHASE + TUNE_PHASE + warmup + steps
+    run_its = STEP_RULE_PHASE + SETTLE_PHASE + warmup + steps
     full_its = fx["iterations"] if fixture_ok else 0
     params = {k: v for k, v in wl.params.items() if k in ("alpha0", "alpha1")}
     params.update({"lambda": lam, "adaptLambda": 0, "dualStorage": dual_kind,
@@ -328,7 +325,7 @@ def cartesian_leg(A, synth, torch, dev, name, batch, dual, steps, warmup, plain=
     def run(engine):
         """(setup s, warmup s, timed s)."""
         out = []
-        for n in (STEP_RULE_PHASE + TUNE_PHASE, warmup, steps):
+        for n in (STEP_RULE_PHASE + SETTLE_PHASE, warmup, steps):
             torch.cuda.synchronize()
             t0 = time.perf_counter()
             for _ in range(n):
@@ -601,7 +598,7 @@ def main():
                    "frames": head["frames"], "coils": head["coils"], "accel": wl.accel,
                    "batch": args.batch, "dual_storage": args.dual, "parallelism": "single-gpu"},
         "protocol": f"each request runs its k<{STEP_RULE_PHASE} step-rule phase and "
-                    f"{TUNE_PHASE} launch-variant timing iterations untimed, then "
+                    f"{SETTLE_PHASE} further iterations untimed, then "
                     f"{args.warmup} warmup + {args.steps} timed steps (k%50==0 step-rule "
                     f"iterations included); full_reconstruction times the whole run",
         "plain_iters_per_s": head["plain_iters_per_s"],

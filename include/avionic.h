@@ -429,8 +429,8 @@ typedef struct avionic_engine_config {
   int voxels_per_lane;      /* dual / primal updates: 1 voxel per lane, or
                                0: a pair of voxels of a row per lane (16- and
                                8-byte accesses) for requests of even width */
-  int fixed_launch;         /* 1: each launch set runs the default launch
-                               variant; 0: a launch set that has run 8 plain
+  int fixed_launch;         /* >= 0: each launch set runs the default launch
+                               variant; < 0: a launch set that has run 8 plain
                                iterations unchanged times its variants (pairs
                                or one voxel per lane; the column pass before
                                or after the dual update; all give the same
