@@ -136,7 +136,7 @@ struct Group {
   int stable = 0, trial = 0;       // plain iterations since the rebuild / timed
   std::vector<int> cands;          // candidate variants of the launch set
   std::vector<float> samples[kVariants];
-  std::array<long, 8> sig{};       // launch-set signature (decision cache key)
+  std::array<long, 10> sig{};      // launch-set signature (decision cache key)
   // Only after a wait for the stream that they were launched on: an event after
   // a launch says that its kernels ran, not that the runtime is done with it.
   void drop_graphs() {
@@ -177,7 +177,7 @@ struct avionic_engine {
   double capture_ms = 0.0;   // host time spent in them
   long long tunings = 0;     // launch sets whose variants were timed
   hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr;  // variant timing
-  std::map<std::array<long, 8>, int> tuned;     // signature -> fastest variant
+  std::map<std::array<long, 10>, int> tuned;    // signature -> fastest variant
   std::map<long long, std::unique_ptr<Slot>> slots;
   std::map<int, Group> groups;  // key = method * 3 + dual storage
 
@@ -276,6 +276,11 @@ struct avionic_engine {
     g.grid.vox = bv;
     g.grid.dp1 = bd1;
     g.grid.dp2 = bd2;
+    g.grid.col = bc;
+    g.grid.row = br;
+    int coils = 1;
+    for (const Slot *s : g.slots) coils = std::max(coils, s->C);
+    g.grid.col_groups = col_coil_groups(bc, coils);
     // launch variants: pairs of voxels unless configured off or no task has
     // an even width (then both lane variants launch the same kernels); the
     // column pass before or after the dual update (two streams only)
@@ -291,12 +296,12 @@ struct avionic_engine {
         g.cands.push_back(variant_of(lanes, first));
       }
     }
-    // signature: the launch set's method, dual storage and the binary orders
-    // of magnitude of its grids (launch sets of similar sizes share a
-    // decision; a serving mix re-times only when its sizes move a lot)
+    // signature: the launch set's method, dual storage, column tiles and the
+    // binary orders of magnitude of its grids (launch sets of similar sizes share
+    // a decision; a serving mix re-times only when its sizes move a lot)
     auto lg = [](long v) { long k = 0; while (v > 1) { v >>= 1; ++k; } return k; };
     g.sig = {g.method, g.ds, lanes0, lg(g.grid.vox), lg(g.grid.col), lg(g.grid.row), lg(bd1),
-             lg(bd2)};
+             lg(bd2), lg(g.grid.col_groups), wide >= kColWideBlocks};
     g.variant = variant_of(lanes0, first0);
     g.tuning = false;
     g.stable = g.trial = 0;
@@ -308,11 +313,6 @@ struct avionic_engine {
       else
         g.tuning = true;
     }
-    g.grid.col = bc;
-    g.grid.row = br;
-    int coils = 1;
-    for (const Slot *s : g.slots) coils = std::max(coils, s->C);
-    g.grid.col_groups = col_coil_groups(bc, coils);
     if (!tasks.empty()) {
       g.table.ensure(sizeof(Task) * tasks.size());
       AV_HIP(hipMemcpyAsync(g.table.p, tasks.data(), sizeof(Task) * tasks.size(),

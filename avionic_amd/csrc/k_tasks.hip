@@ -97,20 +97,23 @@ const char *kernel_name(int id) {
 }
 
 // Column-pass workgroups up to which the column pass is submitted before the
-// dual: 16 per CU, i.e. up to four waves of the 4 resident per CU (the LDS
-// tile).
-static int col_resident_blocks() {
+// dual: 20 per CU, five waves of the 4 resident per CU (the LDS tile).  Measured
+// on MI355X, dual first against column first: 480 workgroups (ICTGV2
+// 256x256x30x16) +5.7%, 3840 (eight of them) +0.5%, 4800 (twelve TGV2
+// 256x256x25x12) +0.7%; 5760 (twelve ICTGV2) -0.2%, 6144 (64 TV 128x128x12x8)
+// -0.6%, 9216 (24 TV 256x256x24x8) -1.0%.
+static int col_first_blocks() {
   static int n = [] {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    return 16 * cus;
+    return 20 * cus;
   }();
   return n;
 }
 
-bool default_col_first(const TaskGrid &gr) { return gr.col < col_resident_blocks(); }
+bool default_col_first(const TaskGrid &gr) { return gr.col <= col_first_blocks(); }
 
 // Dual (primal = false) or primal update over every task, in the grid's
 // launch variant (TaskGrid::lanes).
@@ -196,10 +199,7 @@ void launch_iteration(int method, int ds, const Task *d_tasks, int n, const Task
     // of 256x256x30x16: 480 workgroups; eight: 3840) is submitted first, so
     // that its workgroups start and the dual fills the rest of the CUs; the
     // dual still depends only on what precedes the column pass.  Larger
-    // column passes go after the dual (measured on MI355X, ICTGV2
-    // 256x256x30x16: 1 reconstruction 2507 -> 2724 it/s with this order;
-    // 8 reconstructions 3268 -> 3283 it/s once the dual reads and writes y
-    // with non-temporal accesses, 3219 -> 3172 before).
+    // column passes go after the dual (default_col_first).
     AV_HIP(hipEventRecord(st.fork, s));
     launch_task_col_forward(false, gr, d_tasks, n, s);
     AV_HIP(hipStreamWaitEvent(s2, st.fork, 0));

@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/avionic.h"
@@ -171,6 +172,42 @@ void capture_error() {
   CHECK(avionic_engine_destroy(e) == 0);
 }
 
+// Position of the first launch of a kernel among `v`.
+size_t first_of(const std::vector<std::string> &v, const char *kernel) {
+  size_t i = 0;
+  while (i < v.size() && v[i].find(kernel) == std::string::npos) ++i;
+  CHECK(i < v.size());
+  return i;
+}
+// The launch order by the column pass's grid (before the dual update up to 20
+// blocks per CU; the stand-in has 256 CUs), and decisions of their own for launch
+// sets whose row or column grids differ.
+void launch_sets() {
+  for (const auto &[frames, requests, first] :
+       {std::tuple{8u, 1, true}, {128u, 38, true}, {128u, 41, false}}) {
+    avionic_engine *e = engine(config(0, 1));
+    std::vector<Req> r;
+    for (int i = 0; i < requests; ++i) r.emplace_back(0, frames, 16, 16, 1, 1, 0);
+    long long id = 0;
+    for (Req &q : r) CHECK(q.submit(e, &id) == 0);
+    stub_take_launches();
+    CHECK(avionic_engine_step(e, nullptr) >= 0);
+    const std::vector<std::string> v = stub_take_launches();
+    CHECK((first_of(v, "kt_col_forward") < first_of(v, "kt_dual")) == first);
+    CHECK(avionic_engine_destroy(e) == 0);
+  }
+  avionic_engine_config c = config(1, 1);
+  c.fixed_launch = -1;
+  avionic_engine *e = engine(c);
+  for (unsigned coils : {1u, 8u}) {  // the same voxels, eight times the rows
+    std::vector<Req> r;
+    r.emplace_back(1, 8, 32, 32, coils, 60, 0);
+    run_all(e, r);
+  }
+  CHECK(counts(e).launch_tunings == 2);
+  CHECK(avionic_engine_destroy(e) == 0);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -179,6 +216,7 @@ int main(int argc, char **argv) {
   if (what == "mixed") mixed();
   else if (what == "variants") variants();
   else if (what == "capture_error") capture_error();
+  else if (what == "launch_sets") launch_sets();
   else CHECK(!"a scenario");
   CHECK(stub_launches() > 0);
   CHECK(stub_faults() == 0);

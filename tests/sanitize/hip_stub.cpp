@@ -105,6 +105,11 @@ void put(Stream *s, std::function<void()> f) {
   else
     s->todo.push_back(std::move(f));
 }
+std::map<const void *, std::string> &names() {  // filled before main
+  static auto *m = new std::map<const void *, std::string>;
+  return *m;
+}
+std::vector<std::string> launched;
 void unsafe_in_capture(const char *what) {
   if (building && builder == std::this_thread::get_id()) fault(what);
 }
@@ -117,6 +122,10 @@ size_t stub_memory_held() { return held; }
 size_t stub_memory_peak() { return peak; }
 void stub_reset_peak() { peak = held; }
 long stub_launches() { return launches; }
+std::vector<std::string> stub_take_launches() {
+  std::lock_guard<std::recursive_mutex> l(mu);
+  return std::move(launched);
+}
 long stub_graphs() { return graphs; }
 void stub_fail_launch(long n) { fail_in = n; }
 
@@ -363,12 +372,14 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *sh, hipStream_t *
   *s = cfg_stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3 g, dim3 b, void **, size_t shared, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t shared, hipStream_t s) {
   std::lock_guard<std::recursive_mutex> l(mu);
   if (!g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535) fault("launch grid out of range");
   if (!b.x || b.x * b.y * b.z > 1024) fault("launch block out of range");
   if (shared > 160 * 1024) fault("launch with more LDS than a CU has");
   ++launches;
+  auto it = names().find(f);
+  launched.push_back(it == names().end() ? "?" : it->second);
   if (fail_in > 0 && --fail_in == 0) return fail(hipErrorInvalidValue);
   put(of(s), [] {});
   return hipSuccess;
@@ -377,8 +388,10 @@ void **__hipRegisterFatBinary(const void *) {
   static void *h;
   return &h;
 }
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *,
-                           void *, void *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *,
+                           void *, void *, int *) {
+  names()[f] = name;
+}
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void **) {}
 int roctxRangePushA(const char *) { return 0; }
