@@ -55,7 +55,8 @@ struct Slot {
   int debugstep = 1;
   DevView gap_a, gap_b;
   std::vector<double> gap_log, norm_log, fid_log;
-  size_t bytes = 0;
+  size_t bytes = 0;  // state streamed by an iteration (slot_bytes)
+  size_t held = 0;   // device memory held: bytes, and what its block is larger by
   Task task{};
 
   bool adapts(int k) const {
@@ -642,12 +643,15 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
       layout.add(s->gap_a, sizeof(double) * np);
       layout.add(s->gap_b, sizeof(double) * np);
     }
-    s->mem = PoolBlock(layout.total);
+    // A kept block may be a little larger than the request: what it is larger by
+    // counts against the budget too, and a new block of the exact size is taken
+    // where that would not fit.  The pool gives way to held requests.
+    const size_t left = e->cfg.hbm_budget_bytes - e->used - s->bytes;
+    s->mem = PoolBlock(layout.total, std::min(layout.total / 16, left), left);
     layout.cut(s->mem);
+    s->held = s->bytes + (s->mem.bytes - layout.total);
     s->busy = st;
-    // kept blocks stay within the engine's budget beside the held requests
-    const size_t held = e->used + s->bytes;
-    trim_pool(e->cfg.hbm_budget_bytes > held ? e->cfg.hbm_budget_bytes - held : 0);
+    trim_pool(e->cfg.hbm_budget_bytes - e->used - s->held);
     AV_HIP(hipMemsetAsync(s->x.p, 0, s->x.bytes, st));
     AV_HIP(hipMemsetAsync(s->y.p, 0, s->y.bytes, st));
     AV_HIP(hipMemsetAsync(s->z.p, 0, s->z.bytes, st));
@@ -709,7 +713,7 @@ int avionic_engine_submit(avionic_engine *e, const avionic_request_desc *d, long
 
     s->id = e->next_id++;
     *id = s->id;
-    e->used += s->bytes;
+    e->used += s->held;
     if (s->maxit == 0) {
       s->done = true;
     } else if (runs_now) {
@@ -789,7 +793,7 @@ int avionic_engine_poll(avionic_engine *e, long long id, float *x_out, void *str
     AV_HIP(hipMemcpy(&hs, s->sc.p, sizeof(hs), hipMemcpyDeviceToHost));
     AV_HIP(hipMemcpyAsync(x_out, s->x.p, sizeof(float2) * s->N, hipMemcpyDeviceToDevice, us));
     AV_HIP(hipStreamSynchronize(us));
-    e->used -= s->bytes;
+    e->used -= s->held;
     for (auto &kv : e->groups) {
       auto &v = kv.second.slots;
       auto f = std::find(v.begin(), v.end(), s);
@@ -825,7 +829,7 @@ int avionic_engine_cancel(avionic_engine *e, long long id) {
     auto q = std::find(e->queue.begin(), e->queue.end(), s);
     if (q != e->queue.end()) e->queue.erase(q);
     e->retire(s);
-    e->used -= s->bytes;
+    e->used -= s->held;
     e->slots.erase(it);
   });
 }

@@ -64,16 +64,16 @@ void *device_alloc(size_t bytes) {
   return p;
 }
 
-PoolBlock::PoolBlock(size_t need) {
+PoolBlock::PoolBlock(size_t need, size_t waste, size_t keep) {
   AV_HIP(hipGetDevice(&dev));
   need = need > 0 ? need : 256;
   {
-    // the smallest kept block that wastes at most half of the size asked for
+    // the smallest kept block that is large enough
     Pool &g = pool();
     std::lock_guard<std::mutex> lock(g.mu);
     auto best = g.kept.end();
     for (auto it = g.kept.begin(); it != g.kept.end(); ++it)
-      if (it->dev == dev && it->bytes >= need && it->bytes - need <= need / 2 &&
+      if (it->dev == dev && it->bytes >= need && it->bytes - need <= waste &&
           (best == g.kept.end() || it->bytes < best->bytes))
         best = it;
     if (best != g.kept.end()) {
@@ -83,6 +83,7 @@ PoolBlock::PoolBlock(size_t need) {
       g.kept.erase(best);
       return;
     }
+    trim_locked(g, keep);
   }
   p = device_alloc(need);
   bytes = need;

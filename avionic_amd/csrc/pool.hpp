@@ -20,7 +20,11 @@ constexpr size_t kPoolBytes = size_t(4) << 30;
 class PoolBlock {
  public:
   PoolBlock() = default;
-  explicit PoolBlock(size_t bytes);  // throws when the device has no such memory
+  // Throws when the device has no such memory.  A kept block is taken when it is
+  // at most `waste` bytes larger; for a new one the pool first frees kept blocks
+  // down to `keep` bytes.
+  explicit PoolBlock(size_t bytes) : PoolBlock(bytes, bytes / 2, kPoolBytes) {}
+  PoolBlock(size_t bytes, size_t waste, size_t keep);
   PoolBlock(PoolBlock &&o) noexcept;
   PoolBlock &operator=(PoolBlock &&o) noexcept;
   ~PoolBlock() { give(); }
