@@ -98,6 +98,7 @@ def _declare(L):
     sig = {
         "avionic_last_error": (ctypes.c_char_p, []),
         "avionic_version": (ctypes.c_char_p, []),
+        "avionic_release_memory": (_I, []),
         "avionic_bin_read": (_I, [ctypes.c_char_p, _P, _P, _SZ, ctypes.POINTER(_SZ),
                                   ctypes.POINTER(_I)]),
         "avionic_bin_write": (_I, [ctypes.c_char_p, _P, _P, _SZ]),
@@ -154,6 +155,12 @@ def _check(rc):
 
 def version() -> str:
     return lib().avionic_version().decode()
+
+
+def release_memory():
+    """Gives the device memory that the library keeps idle between
+    reconstructions back to the device, e.g. for torch's allocator."""
+    _check(lib().avionic_release_memory())
 
 
 # ------------------------------------------------------------------ plumbing

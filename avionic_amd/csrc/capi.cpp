@@ -68,6 +68,10 @@ extern "C" {
 const char *avionic_last_error(void) { return g_err.c_str(); }
 const char *avionic_version(void) { return "avionic-mi355x 0.1 (gfx950)"; }
 
+int avionic_release_memory(void) {
+  return guard([&] { trim_pool(0); });
+}
+
 int avionic_cartesian3d_operator_create(unsigned width, unsigned height, unsigned depth,
                                         unsigned coils, const float *mask, avionic_operator **op) {
   return guard([&] {

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "cart_device.hpp"
+#include "pool.hpp"
 
 namespace avionic {
 
@@ -197,7 +198,7 @@ void fft_plan_host(int L, FftPlan &p, std::vector<float2> &tw) {
 void make_fft_plan(int L, FftPlan &p, void **d_tw) {
   std::vector<float2> tw;
   fft_plan_host(L, p, tw);
-  AV_HIP(hipMalloc(d_tw, sizeof(float2) * L));
+  *d_tw = device_alloc(sizeof(float2) * L);
   AV_HIP(hipMemcpy(*d_tw, tw.data(), sizeof(float2) * L, hipMemcpyHostToDevice));
   AV_HIP(hipStreamSynchronize(nullptr));  // landed before any stream reads it
   p.tw = (const float2 *)*d_tw;
@@ -244,8 +245,7 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   has_mask = mask != nullptr;
   std::vector<double> sums((size_t)T * H, 0.0);  // -1: row not sampled
   if (mask) {
-    double *d = nullptr;
-    AV_HIP(hipMalloc((void **)&d, sizeof(double) * sums.size()));
+    double *d = (double *)device_alloc(sizeof(double) * sums.size());
     hipLaunchKernelGGL(k_mask_rows, dim3((unsigned)sums.size()), dim3(NT), 0, s, mask, W, d);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
@@ -299,7 +299,7 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   const size_t o_twx = put(twx.data(), sizeof(float2) * twx.size());
   const size_t o_twy = put(twy.data(), sizeof(float2) * twy.size());
   const size_t o_mrows = host.size();
-  AV_HIP(hipMalloc(&d_tables, o_mrows + sizeof(float) * (size_t)g.nrows * W + 256));
+  d_tables = device_alloc(o_mrows + sizeof(float) * (size_t)g.nrows * W + 256);
   char *base = (char *)d_tables;
   AV_HIP(hipMemcpy(base, host.data(), host.size(), hipMemcpyHostToDevice));
   g.row_off = (const int *)(base + o_off);
@@ -356,8 +356,7 @@ static void launch_cols(float2 *data, const FftPlan &p, int L, int plane, int ba
 void launch_fft2(float2 *data, const FftPlan &pw, const FftPlan &ph, int H, int W, int batch,
                  int sign, int centered, float scale, hipStream_t s) {
   const int RB = pw.ra ? std::min(EMAX / W, NT / pw.ra) : EMAX / W;
-  float2 *tmp = nullptr;
-  AV_HIP(hipMallocAsync((void **)&tmp, sizeof(float2) * (size_t)H * W * batch, s));
+  float2 *tmp = (float2 *)device_alloc_async(sizeof(float2) * (size_t)H * W * batch, s);
   const dim3 grid((H + RB - 1) / RB, batch), block(NT);
   switch (plan_kind(pw, RB)) {
     case kPlanTwo: hipLaunchKernelGGL(k_fft_rows_oop<kPlanTwo>, grid, block, 0, s, data, tmp, pw, H, W, RB, sign, centered); break;

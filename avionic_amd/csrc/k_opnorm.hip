@@ -276,7 +276,7 @@ const Plan64 &plan64(int L) {
     const double a = -2.0 * M_PI * (double)m / (double)L;
     tw[m] = make_double2(std::cos(a), std::sin(a));
   }
-  AV_HIP(hipMalloc((void **)&pl.tw, sizeof(double2) * L));
+  pl.tw = (double2 *)device_alloc(sizeof(double2) * L);
   AV_HIP(hipMemcpy(pl.tw, tw.data(), sizeof(double2) * L, hipMemcpyHostToDevice));
   return g_plans.emplace(std::make_pair(dev, L), pl).first->second;
 }
@@ -492,14 +492,14 @@ void Fp64Scratch::ensure_k(size_t bytes) {
   if (bytes <= k_bytes && k) return;
   if (k) (void)hipFree(k);
   k = nullptr;
-  AV_HIP(hipMalloc(&k, bytes));
+  k = device_alloc(bytes);
   k_bytes = bytes;
 }
 void Fp64Scratch::ensure_red(size_t bytes) {
   if (bytes <= red_bytes && red) return;
   if (red) (void)hipFree(red);
   red = nullptr;
-  AV_HIP(hipMalloc(&red, bytes));
+  red = device_alloc(bytes);
   red_bytes = bytes;
 }
 

@@ -51,17 +51,24 @@ size_t pooled_bytes() {
   return g.bytes;
 }
 
-void *device_alloc(size_t bytes) {
+template <class F>
+static void *alloc_or_trim(size_t bytes, F &&alloc) {
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = alloc(&p);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     trim_pool(0);
-    e = hipMalloc(&p, bytes);
+    e = alloc(&p);
   }
   if (e != hipSuccess)
-    throw Error(-2, std::string("hipMalloc(&p, ") + std::to_string(bytes) + "): " + hipGetErrorString(e));
+    throw Error(-2, "device allocation of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
   return p;
+}
+void *device_alloc(size_t bytes) {
+  return alloc_or_trim(bytes, [&](void **p) { return hipMalloc(p, bytes); });
+}
+void *device_alloc_async(size_t bytes, hipStream_t s) {
+  return alloc_or_trim(bytes, [&](void **p) { return hipMallocAsync(p, bytes, s); });
 }
 
 PoolBlock::PoolBlock(size_t need, size_t waste, size_t keep) {

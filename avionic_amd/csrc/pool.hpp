@@ -5,10 +5,12 @@
 // hipFree waits for the device).  Blocks that are given back are kept, at most
 // kPoolBytes per process, and handed to the next request of a like size on the
 // same device.  They go back to the device when the last solver or engine is
-// destroyed, when the bound is passed (oldest first), and when an allocation
-// fails.  Thread-safe; whoever gives a block back has waited for the streams
+// destroyed, when the bound is passed (oldest first), when an allocation of the
+// library fails, and on request (avionic_release_memory).  Thread-safe; whoever gives a block back has waited for the streams
 // that use it.
 #pragma once
+
+#include <hip/hip_runtime.h>
 
 #include <cstddef>
 
@@ -34,8 +36,10 @@ class PoolBlock {
   int dev = 0;
 };
 
-// hipMalloc that empties the pool and tries again when memory runs out.
+// hipMalloc (stream: hipMallocAsync on it) that empties the pool and tries again
+// when memory runs out; every device allocation of the library goes through them.
 void *device_alloc(size_t bytes);
+void *device_alloc_async(size_t bytes, hipStream_t stream);
 
 // Owners of blocks: the pool is emptied when the last one ends.
 struct PoolUser {

@@ -100,6 +100,11 @@ typedef struct avionic_recon avionic_recon;
 const char *avionic_last_error(void);
 /* Library version string. */
 const char *avionic_version(void);
+/* Gives the device memory that the library keeps idle between reconstructions
+ * (at most 4 GiB while a solver or engine exists) back to the device, for an
+ * allocator beside the library's own; the library's allocations do so by
+ * themselves when memory runs out. */
+int avionic_release_memory(void);
 
 /* ------------------------------------------------------------------------ */
 /* L2 operators (CUDA/include/base_operator.h:24-112)                        */
