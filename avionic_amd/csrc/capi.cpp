@@ -3,6 +3,7 @@
 // message for avionic_last_error().
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -188,8 +189,10 @@ int avionic_recon_create(avionic_method method, unsigned width, unsigned height,
   return guard([&] {
     NEED(recon); NEED(op);
     *recon = nullptr;
-    auto *r = new Recon((int)method, (int)width, (int)height, (int)coils, (int)frames, params, op->op);
-    *recon = new avionic_recon{r};
+    auto r = std::make_unique<Recon>((int)method, (int)width, (int)height, (int)coils, (int)frames,
+                                     params, op->op);
+    *recon = new avionic_recon{r.get()};
+    (void)r.release();
   });
 }
 

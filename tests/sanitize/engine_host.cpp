@@ -4,9 +4,11 @@
 // there, so no result is checked, only what the host does around them.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -21,6 +23,17 @@
       std::exit(1);                                                              \
     }                                                                            \
   } while (0)
+
+// Host allocations of the library: the one that `fail_new` counts down to throws.
+static long fail_new = 0;
+void *operator new(size_t n) {
+  if (fail_new > 0 && !stub_inside() && --fail_new == 0) throw std::bad_alloc();
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void *operator new(size_t n, const std::nothrow_t &) noexcept { return std::malloc(n ? n : 1); }
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -300,6 +313,44 @@ void out_of_memory() {
   stub_set_memory(4096 * kMiB);
 }
 
+// A host allocation that fails anywhere in a reconstruction or a request is an
+// error of that call (or of none): nothing aborts, nothing is lost, and the next
+// call runs.
+void host_memory() {
+  Req q(1, 3, 24, 32, 2, 12, 0);
+  const size_t held = stub_memory_held();
+  long failures = 0;
+  for (long n = 1;; ++n) {
+    avionic_operator *op = nullptr;
+    avionic_recon *r = nullptr;
+    avionic_engine *e = nullptr;
+    avionic_engine_config c = config(1, 4);
+    int rc = 0;
+    fail_new = n;
+    if (!rc) rc = avionic_cartesian_operator_create(32, 24, 2, 3, nullptr, 0, &op);
+    if (!rc) rc = avionic_recon_create(AVIONIC_TGV2, 32, 24, 2, 3, &q.p, op, &r);
+    if (!rc) rc = avionic_recon_run(r, q.data, q.out, q.b1, nullptr);
+    if (!rc) rc = avionic_engine_create(&c, &e);
+    long long id = 0;
+    if (!rc) rc = q.submit(e, &id);
+    while (!rc && avionic_engine_poll(e, id, q.out, nullptr) == 0)
+      rc = std::min(0, avionic_engine_step(e, nullptr));
+    const bool reached = fail_new == 0;
+    fail_new = 0;
+    failures += rc != 0;
+    CHECK(reached || rc == 0);
+    if (r) {  // the solver is as good as before
+      CHECK(avionic_recon_run(r, q.data, q.out, q.b1, nullptr) == 0);
+      CHECK(avionic_recon_destroy(r) == 0);
+    }
+    if (e) CHECK(avionic_engine_destroy(e) == 0);
+    if (op) CHECK(avionic_operator_destroy(op) == 0);
+    CHECK(stub_memory_held() == held && stub_graphs() == 0);
+    if (!reached) break;
+  }
+  CHECK(failures > 20);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -311,6 +362,7 @@ int main(int argc, char **argv) {
   else if (what == "launch_sets") launch_sets();
   else if (what == "budget") budget();
   else if (what == "out_of_memory") out_of_memory();
+  else if (what == "host_memory") host_memory();
   else CHECK(!"a scenario");
   CHECK(stub_launches() > 0);
   CHECK(stub_faults() == 0);

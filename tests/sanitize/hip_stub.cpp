@@ -45,6 +45,17 @@ struct Graph {
 };
 
 std::recursive_mutex mu;
+int inside = 0;  // calls into this file
+struct Guard {
+  Guard() {
+    mu.lock();
+    ++inside;
+  }
+  ~Guard() {
+    --inside;
+    mu.unlock();
+  }
+};
 Stream null_stream;
 std::set<Stream *> streams{&null_stream};
 std::set<void *> execs;
@@ -117,13 +128,14 @@ void unsafe_in_capture(const char *what) {
 }  // namespace
 
 int stub_faults() { return faults; }
+bool stub_inside() { return inside > 0; }
 void stub_set_memory(size_t bytes) { cap = bytes; }
 size_t stub_memory_held() { return held; }
 size_t stub_memory_peak() { return peak; }
 void stub_reset_peak() { peak = held; }
 long stub_launches() { return launches; }
 std::vector<std::string> stub_take_launches() {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   return std::move(launched);
 }
 long stub_graphs() { return graphs; }
@@ -132,7 +144,7 @@ void stub_fail_launch(long n) { fail_in = n; }
 extern "C" {
 
 hipError_t hipMalloc(void **p, size_t n) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   unsafe_in_capture("hipMalloc during a capture");
   if (held + n > cap) return fail(hipErrorOutOfMemory);
   *p = std::calloc(1, n ? n : 1);
@@ -142,7 +154,7 @@ hipError_t hipMalloc(void **p, size_t n) {
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   if (!p) return hipSuccess;
   unsafe_in_capture("hipFree during a capture");
   retire_all();
@@ -159,13 +171,13 @@ hipError_t hipFree(void *p) {
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 hipError_t hipFreeAsync(void *p, hipStream_t) { return hipFree(p); }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   *t = cap;
   *f = cap - held;
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   if (on_device(s)) {
     put(of(st), [=] { std::memcpy(d, s, n); });
   } else {
@@ -175,7 +187,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
   return hipSuccess;
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   unsafe_in_capture("hipMemcpy during a capture");
   retire(&null_stream);
   std::memcpy(d, s, n);
@@ -183,34 +195,34 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
 }
 hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h,
                             hipMemcpyKind, hipStream_t st) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   put(of(st), [=] {
     for (size_t i = 0; i < h; ++i) std::memcpy((char *)d + i * dp, (const char *)s + i * sp, w);
   });
   return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   if (of(st)->capturing) fault("hipMemsetAsync during a capture");
   put(of(st), [=] { std::memset(d, v, n); });
   return hipSuccess;
 }
 hipError_t hipMemset(void *d, int v, size_t n) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   retire(&null_stream);
   std::memset(d, v, n);
   return hipSuccess;
 }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = new Stream;
   streams.insert(p);
   *s = reinterpret_cast<hipStream_t>(p);
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = of(s);
   if (p->capturing) fault("hipStreamDestroy during a capture");
   retire(p);
@@ -221,13 +233,14 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = of(s);
   if (p->capturing) fault("hipStreamSynchronize of a stream that is captured");
   retire(p);
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  Guard l;
   *e = reinterpret_cast<hipEvent_t>(new Event);
   return hipSuccess;
 }
@@ -237,7 +250,7 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t ev, hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Event *e = reinterpret_cast<Event *>(ev);
   e->on = of(s);
   e->captured = e->on->capturing;
@@ -246,7 +259,7 @@ hipError_t hipEventRecord(hipEvent_t ev, hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t ev) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Event *e = reinterpret_cast<Event *>(ev);
   if (e->captured) fault("hipEventSynchronize of a captured event");
   if (e->on && streams.count(e->on)) run(e->on, e->left);
@@ -260,7 +273,7 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) {
   return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t ev, unsigned) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = of(s);
   Event *e = reinterpret_cast<Event *>(ev);
   if (e->captured && building) {
@@ -278,7 +291,7 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t ev, unsigned) {
 }
 
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = of(s);
   if (building || s == nullptr) fault("capture begun inside another, or on the null stream");
   building = new Graph;
@@ -289,7 +302,7 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Stream *p = of(s);
   if (!p->capturing || !p->origin || !building) {
     fault("hipStreamEndCapture without a capture");
@@ -303,7 +316,7 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
   return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   if (fail_in > 0 && --fail_in == 0) return hipErrorInvalidValue;
   Exec *p = new Exec;
   execs.insert(p);
@@ -316,7 +329,7 @@ hipError_t hipGraphDestroy(hipGraph_t g) {
   return hipSuccess;
 }
 hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Exec *p = reinterpret_cast<Exec *>(e);
   if (!execs.count(p)) {
     fault("hipGraphExecDestroy of no executable");
@@ -328,7 +341,7 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
   return hipSuccess;
 }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   Exec *p = reinterpret_cast<Exec *>(e);
   Stream *st = of(s);
   if (!execs.count(p)) fault("hipGraphLaunch of no executable");
@@ -373,7 +386,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *sh, hipStream_t *
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **, size_t shared, hipStream_t s) {
-  std::lock_guard<std::recursive_mutex> l(mu);
+  Guard l;
   if (!g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535) fault("launch grid out of range");
   if (!b.x || b.x * b.y * b.z > 1024) fault("launch block out of range");
   if (shared > 160 * 1024) fault("launch with more LDS than a CU has");

@@ -5,6 +5,7 @@
 #include <vector>
 
 int stub_faults();                       // objections so far
+bool stub_inside();                       // a call of the stand-in is running
 void stub_set_memory(std::size_t bytes);  // device memory from now on
 std::size_t stub_memory_held();
 std::size_t stub_memory_peak();          // since stub_reset_peak

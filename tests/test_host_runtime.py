@@ -53,7 +53,7 @@ def exe(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["mixed", "variants", "capture_error", "launch_sets",
-                                      "budget", "out_of_memory"])
+                                      "budget", "out_of_memory", "host_memory"])
 def test_engine_host(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=240, env=ENV)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
