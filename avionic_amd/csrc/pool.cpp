@@ -4,6 +4,7 @@
 
 #include <deque>
 #include <mutex>
+#include <new>
 #include <string>
 
 #include "common.hpp"
@@ -112,13 +113,17 @@ void PoolBlock::give() {
   if (!p) return;
   Pool &g = pool();
   std::lock_guard<std::mutex> lock(g.mu);
-  if (g.users == 0 || bytes > kPoolBytes) {
-    (void)hipFree(p);
-  } else {
+  bool keep = g.users > 0 && bytes <= kPoolBytes;
+  if (keep) {
     trim_locked(g, kPoolBytes - bytes);
-    g.kept.push_back(Kept{p, bytes, dev});
-    g.bytes += bytes;
+    try {
+      g.kept.push_back(Kept{p, bytes, dev});
+      g.bytes += bytes;
+    } catch (const std::bad_alloc &) {  // this runs in destructors
+      keep = false;
+    }
   }
+  if (!keep) (void)hipFree(p);
   p = nullptr;
 }
 

@@ -349,6 +349,17 @@ void host_memory() {
     if (!reached) break;
   }
   CHECK(failures > 20);
+  // blocks given back with no host memory to note them
+  avionic_engine *e = engine(config(0, 1));
+  std::vector<long long> id(60);
+  for (long long &i : id) CHECK(q.submit(e, &i) == 0);
+  for (long long i : id) {
+    fail_new = 1;
+    avionic_engine_cancel(e, i);
+    fail_new = 0;
+  }
+  CHECK(counts(e).held == 0);
+  CHECK(avionic_engine_destroy(e) == 0);
 }
 
 }  // namespace
