@@ -488,7 +488,7 @@ __host__ __device__ constexpr int col_table_len(int kind) {
   return kind & 1 ? kTwoMaxLen : (kind == 2 ? kMaxFftLen : kMaxFftLenNarrow);
 }
 __host__ __device__ constexpr int row_table_len(int kind) {
-  return kind == 0 ? kTwoMaxLen : (kind == 2 ? kMaxFftLen : kMaxFftLenNarrow);
+  return kind == kRowTwo || kind == kRow256 ? kTwoMaxLen : (kind == kRowWide ? kMaxFftLen : kMaxFftLenNarrow);
 }
 
 }  // namespace avionic

@@ -30,7 +30,7 @@ struct CartGeom {
   int XB, lxb, nxb;  // columns per column-pass tile (two-stage: 2^lxb), tiles
   int RB;            // rows per row-pass block
   int lja, ljb;      // two-stage: log2 of the lanes per row in the radix-ra / -rb stages
-  int wide_col, wide_row;  // column / row plan is wide (plan_is_wide)
+  int ckind, rkind;  // kernels that run it (ColKind, RowKind)
   long nrows;          // sampled rows over all frames (row_off[T])
   long nrows_c;        // C * nrows
   const int *row_off;  // [T+1]
@@ -42,17 +42,14 @@ struct CartGeom {
   FftPlan pw, ph;
 };
 
-// Kind of a geometry's column passes (one kernel per kind): 0 runtime plan,
-// 1 two-stage (cart_two.hpp), 2 wide runtime plan, 3 two-stage, length 256.
+// Kernels of the column passes: runtime plan, two-stage (cart_two.hpp), wide
+// runtime plan, two-stage with the constants of length 256.
+enum ColKind { kColRt = 0, kColTwo = 1, kColWide = 2, kCol256 = 3 };
 constexpr int kColKinds = 4;
-__host__ __device__ inline int col_kind(const CartGeom &g) {
-  return g.ph.ra ? (g.ph.L == 256 && g.lxb == 4 ? 3 : 1) : (g.wide_col ? 2 : 0);
-}
-// Kind of the row pass: 0 two-stage, 1 runtime plan, 2 wide runtime plan.
-constexpr int kRowKinds = 3;
-__host__ __device__ inline int row_kind(const CartGeom &g) {
-  return g.pw.ra ? 0 : (g.wide_row ? 2 : 1);
-}
+// Kernels of the row pass: two-stage, runtime plan, wide runtime plan, and the
+// two-stage one of the engine without a bound on its registers (length 256).
+enum RowKind { kRowTwo = 0, kRowRt = 1, kRowWide = 2, kRow256 = 3 };
+constexpr int kRowKinds = 4;
 
 // Row-pass modes.
 enum RowMode {  // Norm2, Residual: one partial sum per row block

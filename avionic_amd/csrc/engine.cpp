@@ -155,6 +155,19 @@ struct Group {
   }
 };
 
+// Two-stage row tasks of one launch set run in one kernel (kernels of one pass
+// run one after the other, each with a tail of its own): the one of the larger
+// part.  The bits are the same.
+void merge_row_kinds(const std::vector<Slot *> &slots) {
+  long row[kRowKinds] = {};
+  for (const Slot *s : slots)
+    if (s->cart) row[s->task.cg.rkind] += s->task.nrow_blocks;
+  if (!row[kRowTwo] || !row[kRow256]) return;
+  const int from = row[kRowTwo] > row[kRow256] ? kRow256 : kRowTwo;
+  for (Slot *s : slots)
+    if (s->cart && s->task.cg.rkind == from) s->task.cg.rkind = from == kRow256 ? kRowTwo : kRow256;
+}
+
 }  // namespace
 
 struct avionic_engine {
@@ -235,12 +248,6 @@ struct avionic_engine {
     // are destroyed, and the task table rewritten, only once they are done.
     AV_HIP(hipStreamSynchronize(stream));
     g.drop_graphs();
-    // tasks ordered by column kind, then row kind: each kind's kernel is
-    // launched over its own span of blocks only
-    std::stable_sort(g.slots.begin(), g.slots.end(), [&](const Slot *a, const Slot *b) {
-      const int ka = col_kind(a->task.cg), kb = col_kind(b->task.cg);
-      return ka != kb ? ka < kb : row_kind(a->task.cg) < row_kind(b->task.cg);
-    });
     // column tiles by the launch set's size (the results do not depend on them)
     long wide = 0;
     for (const Slot *s : g.slots)
@@ -248,8 +255,16 @@ struct avionic_engine {
     for (Slot *s : g.slots)
       if (s->cart) {
         set_col_tiles(s->task.cg, wide >= kColWideBlocks);
+        set_row_tiles(s->task.cg, true);
         s->task.ncol_blocks = s->task.cg.nxb * s->task.cg.T;
       }
+    merge_row_kinds(g.slots);
+    // tasks ordered by column kind, then row kind: each kind's kernel is
+    // launched over its own span of blocks only
+    std::stable_sort(g.slots.begin(), g.slots.end(), [&](const Slot *a, const Slot *b) {
+      const int ka = a->task.cg.ckind, kb = b->task.cg.ckind;
+      return ka != kb ? ka < kb : a->task.cg.rkind < b->task.cg.rkind;
+    });
     std::vector<Task> tasks;
     int bv = 0, bd1 = 0, bd2 = 0, bc = 0, br = 0;
     g.grid = TaskGrid{};
@@ -261,7 +276,7 @@ struct avionic_engine {
       t.b_dp2 = bd2;
       t.b_col = bc;
       t.b_row = br;
-      const int ck = col_kind(t.cg), rk = row_kind(t.cg);
+      const int ck = t.cg.ckind, rk = t.cg.rkind;
       if (!col_seen[ck]) g.grid.col_lo[ck] = bc;
       if (!row_seen[rk]) g.grid.row_lo[rk] = br;
       col_seen[ck] = row_seen[rk] = true;

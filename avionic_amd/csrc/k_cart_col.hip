@@ -67,9 +67,9 @@ static void col_fwd(int kind, const CartGeom &g, const float2 *u, const float2 *
 void launch_col_forward(const CartGeom &g, const float2 *u, const float2 *usub, const float2 *b1,
                         float2 *kcol, hipStream_t s) {
   if (usub)
-    col_fwd<true>(col_kind(g), g, u, usub, b1, kcol, s);
+    col_fwd<true>(g.ckind, g, u, usub, b1, kcol, s);
   else
-    col_fwd<false>(col_kind(g), g, u, usub, b1, kcol, s);
+    col_fwd<false>(g.ckind, g, u, usub, b1, kcol, s);
 }
 
 template <class P, int G>
@@ -99,7 +99,7 @@ static void col_adj_groups(const CartGeom &g, const float2 *zhat, const float2 *
 void launch_col_adjoint(const CartGeom &g, const float2 *zhat, const float2 *b1, float2 *out,
                         hipStream_t s) {
   const dim3 grid(g.nxb, g.T), block(NT);
-  switch (col_kind(g)) {
+  switch (g.ckind) {
     case 0: hipLaunchKernelGGL(k_col_adjoint_rt<false>, grid, block, 0, s, g, zhat, b1, out); break;
     case 2: hipLaunchKernelGGL(k_col_adjoint_rt<true>, grid, block, 0, s, g, zhat, b1, out); break;
     case 1: col_adj_groups<TwoRt>(g, zhat, b1, out, s); break;

@@ -40,9 +40,10 @@ static void launch_row_kind(const CartGeom &g, int nb, const float2 *kcol, float
                             const float2 *d, float2 *zhat, float2 *out, const float2 *zin,
                             const DevScalars *sc, double *partial, hipStream_t s) {
   const dim3 grid(nb), block(NT);
-  switch (row_kind(g)) {
-    case 0: hipLaunchKernelGGL((k_row_pass<MODE, 0>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
-    case 1: hipLaunchKernelGGL((k_row_pass<MODE, 1>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
+  switch (g.rkind) {
+    case kRowTwo:
+    case kRow256: hipLaunchKernelGGL((k_row_pass<MODE, 0>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
+    case kRowRt: hipLaunchKernelGGL((k_row_pass<MODE, 1>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
     default: hipLaunchKernelGGL((k_row_pass<MODE, 2>), grid, block, 0, s, g, kcol, z, d, zhat, out, zin, sc, partial); break;
   }
 }

@@ -117,15 +117,21 @@ void set_col_tiles(CartGeom &g, bool wide) {
   g.XB = col_tile(g, wide);
   g.lxb = log2_ceil(g.XB);
   g.nxb = (g.W + g.XB - 1) / g.XB;
+  if (g.ph.ra)
+    g.ckind = g.ph.L == 256 && g.lxb == 4 ? kCol256 : kColTwo;
+  else
+    g.ckind = plan_is_wide(g.ph) ? kColWide : kColRt;
 }
 void set_row_tiles(CartGeom &g, bool wide) {
   if (!g.pw.ra) {
     g.RB = std::max(1, std::min(kRowMaxRows, kRowTileElems / g.W));
+    g.rkind = plan_is_wide(g.pw) ? kRowWide : kRowRt;
     return;
   }
   g.ljb = log2_ceil(g.pw.ra);
   g.lja = wide ? std::max(log2_ceil(g.pw.rb), g.ljb - log2_ceil(two_most(g.pw.rb))) : g.ljb;
   g.RB = NT >> g.lja;
+  g.rkind = g.pw.L == 256 ? kRow256 : kRowTwo;
 }
 long wide_col_blocks(const CartGeom &g) {
   const int xb = col_tile(g, true);
@@ -317,8 +323,6 @@ void CartPlan::init(int W, int H, int C, int T, const float *mask, int centered,
   set_col_tiles(g, wide_col_blocks(g) >= kColWideBlocks);
   set_row_tiles(g, true);
   if (row_blocks() < kRowWideBlocks) set_row_tiles(g, false);
-  g.wide_col = plan_is_wide(g.ph) ? 1 : 0;
-  g.wide_row = plan_is_wide(g.pw) ? 1 : 0;
   // The tables above come from pageable host memory (such a copy, on the null
   // stream, may return before its data has landed) and from a kernel there, and
   // the kernels that index with them may run on non-blocking streams, which do

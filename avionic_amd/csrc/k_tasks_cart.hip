@@ -1,6 +1,6 @@
 // Task-list column and row passes of the Cartesian operator (tasks.hpp).
 //
-// One kernel per kind of plan (col_kind, row_kind); a launch covers its kind's
+// One kernel per kind of plan (ColKind, RowKind); a launch covers its kind's
 // span of blocks and is made only when such a task is resident.  DELTA =
 // false: K of the extragradient image (dual update); DELTA = true: K of
 // ext - x (step rule, adapting tasks only).  The forward column pass of a
@@ -18,7 +18,7 @@ __global__ __launch_bounds__(NTC) void kt_col_forward(const Task *__restrict__ t
   __shared__ int rml[col_table_len(KIND)];
   const int blk = blk0 + (int)blockIdx.x;
   const Task &T = tasks[find_task<kCol>(tasks, n, blk)];
-  if (col_kind(T.cg) != KIND) return;
+  if (T.cg.ckind != KIND) return;
   if (!task_active(T.sc)) return;
   if (DELTA && !task_adapt(T.sc)) return;
   const int lb = blk - T.b_col, xbi = lb % T.cg.nxb, t = lb / T.cg.nxb;
@@ -34,9 +34,18 @@ __global__ __launch_bounds__(NTC) void kt_col_forward(const Task *__restrict__ t
                                         twl, rml);
 }
 
+// A lane holds the values of its butterflies with z and d beside them: 175 VGPRs,
+// two waves per SIMD.  kRowTwo is held to three waves (168 VGPRs, a little of the
+// largest radices spilled); at 16 x 16 the spill costs more than the wave, so
+// length 256 has its own kernel of the same source (and bits).  Measured on
+// MI355X, without the bound / with it: 64 TV 128x128x12x8 123 -> 119 us (the
+// compile-time pass for 128 before: 114), 64 TV 96x96x8x6 50 -> 44, 32 TV
+// 160x128x12x8 77 -> 68, 16 TGV2 192x160x16x8 69 -> 62, 16 TV 240x128x12x8
+// 55 -> 51; 8 ICTGV2 256x256x30x16 168 -> 176.
 template <int MODE, int RK>
-__global__ __launch_bounds__(NT) void kt_row(const Task *__restrict__ tasks, int n, int blk0) {
-  constexpr bool TWO = RK == 0;
+__global__ __launch_bounds__(NT, RK == kRowTwo ? 3 : 1) void kt_row(const Task *__restrict__ tasks,
+                                                                    int n, int blk0) {
+  constexpr bool TWO = RK == kRowTwo || RK == kRow256;
   __shared__ float2 tile[TWO ? kRowTwoElems : RTILE];
   __shared__ float2 tile2[(MODE == kRowDualUpdate && !TWO) ? RTILE : 1];
   __shared__ float2 twl[row_table_len(RK)];
@@ -44,7 +53,7 @@ __global__ __launch_bounds__(NT) void kt_row(const Task *__restrict__ tasks, int
   __shared__ int mrl[TWO ? 1 : kRowMaxRows];
   const int blk = blk0 + (int)blockIdx.x;
   const Task &T = tasks[find_task<kRow>(tasks, n, blk)];
-  if (row_kind(T.cg) != RK) return;
+  if (T.cg.rkind != RK) return;
   if (!task_active(T.sc)) return;
   if (MODE == kRowNorm2 && !task_adapt(T.sc)) return;
   const int lb = blk - T.b_row;
@@ -52,10 +61,10 @@ __global__ __launch_bounds__(NT) void kt_row(const Task *__restrict__ tasks, int
   if constexpr (TWO)
     a = row_two<MODE>(T.cg, lb, T.kcol, T.z, T.d, T.zhat, nullptr, nullptr, T.sc, tile, twl);
   else if constexpr (MODE == kRowDualUpdate)
-    row_dual_fused<RK == 2>(T.cg, lb, T.kcol, T.z, T.d, T.zhat, T.sc, tile, tile2, twl, mrl);
+    row_dual_fused<RK == kRowWide>(T.cg, lb, T.kcol, T.z, T.d, T.zhat, T.sc, tile, tile2, twl, mrl);
   else
-    a = row_mode_fused<MODE, RK == 2>(T.cg, lb, T.kcol, nullptr, nullptr, nullptr, nullptr, tile,
-                                      twl, mrl);
+    a = row_mode_fused<MODE, RK == kRowWide>(T.cg, lb, T.kcol, nullptr, nullptr, nullptr, nullptr,
+                                             tile, twl, mrl);
   if (MODE == kRowNorm2) {
     a = block_sum(a, red);
     if (threadIdx.x == 0) T.part_k[lb] = a;
@@ -74,7 +83,7 @@ void kt_col_adjoint(const Task *__restrict__ tasks, int n, int blk0) {
   __shared__ int rml[col_table_len(KIND)];
   const int blk = blk0 + (int)blockIdx.x;
   const Task &T = tasks[find_task<kCol>(tasks, n, blk)];
-  if (col_kind(T.cg) != KIND) return;
+  if (T.cg.ckind != KIND) return;
   if (!task_active(T.sc)) return;
   const int lb = blk - T.b_col, xbi = lb % T.cg.nxb, t = lb / T.cg.nxb;
   if constexpr (KIND == 1)

@@ -61,8 +61,8 @@ struct TaskGrid {
   // col_first 1 submits the column pass before the dual update, 0 after it,
   // -1 decides by the column pass's grid size.
   int lanes = 2, col_first = -1;
-  // Blocks [lo, hi) spanning the tasks of each column kind (col_kind) and of
-  // each row kind (row_kind); the engine orders its tasks by kind, so each
+  // Blocks [lo, hi) spanning the tasks of each column kind (ColKind) and of
+  // each row kind (RowKind); the engine orders its tasks by kind, so each
   // span holds only that kind's blocks.
   int col_lo[kColKinds] = {}, col_hi[kColKinds] = {};
   int row_lo[kRowKinds] = {}, row_hi[kRowKinds] = {};
