@@ -168,6 +168,23 @@ void merge_row_kinds(const std::vector<Slot *> &slots) {
     if (s->cart && s->task.cg.rkind == from) s->task.cg.rkind = from == kRow256 ? kRowTwo : kRow256;
 }
 
+// Column tasks of length 256 leave their kernel of compile-time radices for the
+// other two-stage tasks' one (the same bits) where they have fewer than six
+// blocks per CU: two kernels, one after the other, then cost more than the
+// constants save.  Iteration, merged / separate: TGV2 256x256x25x12 (400 blocks)
+// with one or three 192x192x20x10 (240 each) 0.85 / 0.94, two or three with one
+// or three 0.91 / 0.99; four ICTGV2 256x256x30x16 (1920) with four 224x224x24x16
+// 1.01, eight (3840) with one 128x128 1.04.
+constexpr long kCol256Blocks = 1536;
+void merge_col_kinds(const std::vector<Slot *> &slots) {
+  long col[kColKinds] = {};
+  for (const Slot *s : slots)
+    if (s->cart) col[s->task.cg.ckind] += s->task.ncol_blocks;
+  if (!col[kColTwo] || col[kCol256] >= kCol256Blocks) return;
+  for (Slot *s : slots)
+    if (s->cart && s->task.cg.ckind == kCol256) s->task.cg.ckind = kColTwo;
+}
+
 }  // namespace
 
 struct avionic_engine {
@@ -258,6 +275,7 @@ struct avionic_engine {
         set_row_tiles(s->task.cg, true);
         s->task.ncol_blocks = s->task.cg.nxb * s->task.cg.T;
       }
+    merge_col_kinds(g.slots);
     merge_row_kinds(g.slots);
     // tasks ordered by column kind, then row kind: each kind's kernel is
     // launched over its own span of blocks only

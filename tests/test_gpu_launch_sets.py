@@ -42,3 +42,17 @@ def test_row_kernels(gpu, sizes, centered):
     for s, x in zip(sizes, _run(gpu.A, torch, sizes, centered)):
         assert np.isfinite(x).all()
         assert np.array_equal(x, _run(gpu.A, torch, [s], centered)[0]), s
+
+
+# columns of 256 beside other two-stage columns: few, in the kernel of those; and
+# 1600 blocks of them, in their own
+@pytest.mark.parametrize("sizes", [
+    [(39, 256, 3, 3), (96, 192, 3, 2), (33, 225, 2, 2)],
+    [(256, 256, 100, 1), (64, 256, 4, 3), (80, 128, 3, 2)]])
+@pytest.mark.parametrize("centered", [False, True])
+def test_column_kernels(gpu, sizes, centered):
+    import torch
+    print(f"[gpu launch sets] columns {sizes} centered={centered}", flush=True)
+    for s, x in zip(sizes, _run(gpu.A, torch, sizes, centered)):
+        assert np.isfinite(x).all()
+        assert np.array_equal(x, _run(gpu.A, torch, [s], centered)[0]), s
