@@ -97,18 +97,19 @@ const char *kernel_name(int id) {
 }
 
 // Column-pass workgroups up to which the column pass is submitted before the
-// dual: 20 per CU, five waves of the 4 resident per CU (the LDS tile).  Measured
+// dual: 24 per CU, six waves of the 4 resident per CU (the LDS tile).  Measured
 // on MI355X, dual first against column first: 480 workgroups (ICTGV2
 // 256x256x30x16) +5.7%, 3840 (eight of them) +0.5%, 4800 (twelve TGV2
-// 256x256x25x12) +0.7%; 5760 (twelve ICTGV2) -0.2%, 6144 (64 TV 128x128x12x8)
-// -0.6%, 9216 (24 TV 256x256x24x8) -1.0%.
+// 256x256x25x12) +0.7%, 5520 (with three 192x192x20x10) +1.5%, 5760 (twelve
+// ICTGV2) -0.2%, 6144 (64 TV 128x128x12x8) -0.6%, 7680 (sixteen ICTGV2) -0.1%,
+// 9216 (24 TV 256x256x24x8) -1.0%.
 static int col_first_blocks() {
   static int n = [] {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    return 20 * cus;
+    return 24 * cus;
   }();
   return n;
 }

@@ -192,12 +192,12 @@ size_t first_of(const std::vector<std::string> &v, const char *kernel) {
   CHECK(i < v.size());
   return i;
 }
-// The launch order by the column pass's grid (before the dual update up to 20
+// The launch order by the column pass's grid (before the dual update up to 24
 // blocks per CU; the stand-in has 256 CUs), and decisions of their own for launch
 // sets whose row or column grids differ.
 void launch_sets() {
   for (const auto &[frames, requests, first] :
-       {std::tuple{8u, 1, true}, {128u, 38, true}, {128u, 41, false}}) {
+       {std::tuple{8u, 1, true}, {128u, 47, true}, {128u, 49, false}}) {
     avionic_engine *e = engine(config(0, 1));
     std::vector<Req> r;
     for (int i = 0; i < requests; ++i) r.emplace_back(0, frames, 16, 16, 1, 1, 0);
