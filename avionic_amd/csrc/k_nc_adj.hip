@@ -25,8 +25,9 @@ struct NcColAdjStore {
 // centre (a hundred entries) then cost LDS reads, not a chain of dependent
 // global loads on one lane.  The sums keep each cell's entry order, so every
 // application gives the same bits.
-// NZ coils of a frame per block (3 in the compiled kernels; 2 and 4 measured
-// slower at the 256x256x30x12 radial geometry): the tile's offsets are
+// NZ coils of a frame per block (3 in the compiled kernels, 2 at grid length 512;
+// 2 and 4 measured slower than 3 at the 256x256x30x12 radial geometry;
+// nc_adj_coils on runtime plans): the tile's offsets are
 // staged and its entries loaded once for all of them, each entry's products
 // of the NZ coils sit in NZ parts of the tile, and the transforms run one
 // after the other.  Every coil's sums are the one-coil
@@ -199,19 +200,38 @@ void nc_adjoint_ct(const NcGeom &g, const float2 *z, const float2 *b1, float2 *t
   AV_LAUNCH_CHECK();
 }
 
+// Coils per adjoint column block on a runtime plan.  Two share the tile's tables,
+// which pays where one coil per block already makes more than eleven blocks per
+// CU; below that it only lengthens the chain.  Measured on MI355X, K^H with two
+// coils against one (grid length, one-coil blocks): 288 (432) +23%, 336 (2016)
+// +7%, 400 (2400) +1%, 448 (2688) +1%, 504 (3024) -4%, 288 (4608) -2%, 320 (5120)
+// -6%, 448 (13440) -10%.  Two-stage grids: 225 to 240 +4 to +18%, 200 -4 to +26%.
+// Wide kernels, whose two-coil form holds more registers, gain only on tiles of
+// more than 3264 cells: 312 +9 to +23%, 528 to 792 +2 to +15%, 840 to 1024 -8 to
+// -13% (1440 blocks: +2%).
+int nc_adj_coils(int kind, const NcGeom &g, int nXa) {
+  if ((long)nXa * g.T * g.C <= 2816) return 1;
+  return kind == kPlanNarrow || g.XBa * g.Gy > 3264 ? 2 : 1;
+}
+
 // On the geometry's runtime plans.
-template <int KIND>
-void nc_adjoint_rt(const NcGeom &g, const float2 *z, const float2 *b1, float2 *tmp, float2 *img,
-                   hipStream_t s) {
+template <int KIND, int NZ>
+void nc_col_adj_rt(const NcGeom &g, int nXa, const float2 *z, float2 *tmp, hipStream_t s) {
   const size_t cps_bytes = sizeof(int) * ((size_t)g.XBa * g.Gy + 1);
-  const int nXa = (g.Gx + g.XBa - 1) / g.XBa;
-  // two coils per block where the transform has three stages (K^H 224x224x16x8
-  // at osf 2: 186 -> 178 us); two-stage ones lose more blocks than they save
-  // table loads (160x160x24x10 at osf 1.5: 152 -> 157 us)
-  constexpr int NZ = KIND == kPlanTwo ? 1 : 2;
   hipLaunchKernelGGL((k_nc_col_adj<KIND, NcPlanRt, NZ>), dim3(nXa, g.T * ((g.C + NZ - 1) / NZ)),
                      dim3(NCC), cps_bytes, s, g, z, tmp);
   AV_LAUNCH_CHECK();
+}
+template <int KIND>
+void nc_adjoint_rt(const NcGeom &g, const float2 *z, const float2 *b1, float2 *tmp, float2 *img,
+                   hipStream_t s) {
+  const int nXa = (g.Gx + g.XBa - 1) / g.XBa;
+  if constexpr (KIND == kPlanTwo)
+    nc_col_adj_rt<KIND, 1>(g, nXa, z, tmp, s);
+  else if (nc_adj_coils(KIND, g, nXa) == 1)
+    nc_col_adj_rt<KIND, 1>(g, nXa, z, tmp, s);
+  else
+    nc_col_adj_rt<KIND, 2>(g, nXa, z, tmp, s);
   hipLaunchKernelGGL((k_nc_row_adj<KIND, NcPlanRt>), dim3((g.H + g.RBa - 1) / g.RBa, g.T), dim3(NCR),
                      0, s, g, (const float2 *)tmp, b1, img);
   AV_LAUNCH_CHECK();

@@ -23,8 +23,8 @@
 //   3. sample pass: the partials of a point, scaled, feed K u (or the z
 //      update, or a norm reduction).
 // K^H as two passes:
-//   1. column pass (grid (ceil(Gx/XB), T*C); the compiled kernels take three
-//      coils of a frame per block): the spreading, by gathers without
+//   1. column pass (grid (ceil(Gx/XB), T*C); the kernels take up to three coils
+//      of a frame per block): the spreading, by gathers without
 //      atomics: the lanes form the products of the column tile's cell ->
 //      point entries (tce) into LDS, each grid cell sums its own in entry
 //      order; length-Gy inverse transform, keeps the H image rows ->
