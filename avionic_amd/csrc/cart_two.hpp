@@ -1,5 +1,6 @@
 // Two-stage Cartesian passes: transforms whose length is a product of two
-// radices of at most 16 (FftPlan::ra >= rb), i.e. nearly every length up to 256.
+// radices of at most 16 (FftPlan::ra >= rb): every supported length below 125 and
+// 53 of the 69 from 64 to 256.
 //
 // Stage a takes elements j + r rb (r < ra) of butterfly j < rb, stage b
 // elements j + r ra (r < rb) of butterfly j < ra, which are also its output
@@ -14,9 +15,9 @@
 // the chain load -> stage -> barrier -> stage of each coil.  Measured on MI355X
 // against the passes that moved every coil through LDS on a runtime plan (the
 // operator calls before): K at 256 x 256 x 30 frames x 16 coils, acceleration
-// 12, 291 -> 110 us (column pass 228 -> 62 us); K^H at 180 x 240 x 20 x 12,
-// 191 -> 53 us; at 100 x 80 x 4 x 4, 71 -> 16.5 us; one eager TGV2 iteration
-// at 256 x 256 x 25 x 12, 425 -> 220 us.
+// 12, 291 -> 99 us (column pass 228 -> 49 us); K^H at 180 x 240 x 20 x 12,
+// 191 -> 35 us; at 100 x 80 x 4 x 4, 71 -> 12.7 us; one eager TGV2 iteration
+// at 256 x 256 x 25 x 12, 425 -> 184 us.
 #pragma once
 
 #include "cart_fused.hpp"

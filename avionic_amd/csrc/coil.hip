@@ -254,8 +254,8 @@ __global__ void k_ut_pre(const float2 *__restrict__ b1, const float2 *__restrict
 // pixel in each direction, so after them the inner CORE x CORE pixels are the
 // ones the whole image would have given; the block writes those to the other
 // half of a double buffer.  The loops were bound by launches (4 us each, two per
-// iteration): coil estimation at 192 x 160, 12 frames, 6 coils, 38 -> 11
-// ms (the two-kernel conjugate gradients above included).
+// iteration): coil estimation at 192 x 160, 12 frames, 6 coils, 38 -> 10.6
+// to 12.5 ms, by process (the two-kernel conjugate gradients above included).
 constexpr int kHalo = 8;
 // Region side REG, lanes per block, pixels per lane (ROW rows apart).
 template <int REG_>

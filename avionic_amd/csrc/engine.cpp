@@ -92,12 +92,11 @@ inline int variant_col_first(int v) { return (v & 1) ? 0 : 1; }
 inline int variant_of(int lanes, bool col_first) { return (lanes == 1 ? 2 : 0) + (col_first ? 0 : 1); }
 // Variant timing (fixed_launch < 0): a launch set is timed once it has run this
 // many plain iterations unchanged, over this many plain iterations per candidate.
-// Measured over 18 launch sets of all methods (64 x 64 to 320 x 300, 1 to 64
-// requests), pairs with the column pass first are within 1% of the fastest
-// variant, except 64 TV requests of 128 x 128 x 12 x 8 (one voxel per lane 4%
-// faster): too little for a timed phase in every launch set by default, which
-// holds the host and two more captures per variant, and during which two runs
-// of tests once ended in a host abort whose cause is not established.
+// Measured over 41 launch sets of all methods (64 x 64 to 320 x 300, 1 to 128
+// requests), pairs with the default order are within about 2% of the fastest
+// variant: too little for a timed phase in every launch set by default, which
+// holds the host and two more captures per variant, and during which two runs of
+// tests ended in a host abort whose cause is not established.
 constexpr int kTuneAfter = 8, kTuneSamples = 3;
 
 // A stream capture and its graph; an exception on the way ends the capture, so
