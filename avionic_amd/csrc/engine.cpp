@@ -99,13 +99,14 @@ inline int variant_of(int lanes, bool col_first) { return (lanes == 1 ? 2 : 0) +
 // tests ended in a host abort whose cause is not established.
 constexpr int kTuneAfter = 8, kTuneSamples = 3;
 
-// A stream capture and its graph; an exception on the way ends the capture, so
-// that the engine's streams can be used again.
+// A stream capture and its graph; an exception on the way joins the side stream
+// and ends the capture, so that the engine's streams can be used again.
 struct Capture {
-  hipStream_t stream;
+  hipStream_t stream, side;
+  hipEvent_t joined;
   hipGraph_t graph = nullptr;
   bool open = true;
-  explicit Capture(hipStream_t s) : stream(s) {
+  Capture(hipStream_t s, hipStream_t s2, hipEvent_t join) : stream(s), side(s2), joined(join) {
     AV_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   }
   Capture(const Capture &) = delete;
@@ -116,6 +117,10 @@ struct Capture {
   }
   ~Capture() {
     if (open) {
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      if (side && hipStreamIsCapturing(side, &st) == hipSuccess && st == hipStreamCaptureStatusActive &&
+          hipEventRecord(joined, side) == hipSuccess)
+        (void)hipStreamWaitEvent(stream, joined, 0);
       (void)hipStreamEndCapture(stream, &graph);
       (void)hipGetLastError();
     }
@@ -442,7 +447,7 @@ struct avionic_engine {
       if (!ex) {
         TraceRange tr("avionic_engine_capture");
         const auto t0 = std::chrono::steady_clock::now();
-        Capture cap(stream);
+        Capture cap(stream, side, ev_join);
         launch_iteration(g.method, g.ds, g.table.as<Task>(), n, gr, with_step, st, hooks);
         cap.end();
         AV_HIP(hipGraphInstantiate(&ex, cap.graph, nullptr, nullptr, 0));

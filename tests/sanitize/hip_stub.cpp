@@ -31,6 +31,7 @@ struct Exec {
 struct Event;
 struct Stream {
   bool capturing = false, origin = false;
+  bool unjoined = false;  // captured work that the origin does not wait for
   std::deque<std::function<void()>> todo;
   std::vector<Exec *> launched;
 };
@@ -111,10 +112,12 @@ bool on_device(const void *p) {
 }
 // An operation on a stream: a node while it is captured.
 void put(Stream *s, std::function<void()> f) {
-  if (s->capturing)
+  if (s->capturing) {
     ++building->nodes;
-  else
+    s->unjoined = !s->origin;
+  } else {
     s->todo.push_back(std::move(f));
+  }
 }
 std::map<const void *, std::string> &names() {  // filled before main
   static auto *m = new std::map<const void *, std::string>;
@@ -278,9 +281,10 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t ev, unsigned) {
   Event *e = reinterpret_cast<Event *>(ev);
   if (e->captured && building) {
     if (!p->capturing) {
-      p->capturing = true;
+      p->capturing = p->unjoined = true;
       joined.push_back(p);
     }
+    if (p->origin && e->on) e->on->unjoined = false;
     return hipSuccess;
   }
   if (p->capturing) fault("captured stream waits for an event from outside the capture");
@@ -308,11 +312,19 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
     fault("hipStreamEndCapture without a capture");
     return fail(hipErrorInvalidValue);
   }
-  for (Stream *j : joined) j->capturing = false;
+  for (Stream *j : joined) {
+    if (j->unjoined) fault("hipStreamEndCapture with a stream that was not joined");
+    j->capturing = j->unjoined = false;
+  }
   joined.clear();
   p->capturing = p->origin = false;
   *g = reinterpret_cast<hipGraph_t>(building);
   building = nullptr;
+  return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st) {
+  Guard l;
+  *st = of(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
