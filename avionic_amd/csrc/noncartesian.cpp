@@ -170,6 +170,8 @@ class NoncartesianOperator : public Operator {
       if (d < -1e-12) return J * std::sin(std::sqrt(-d)) / std::sqrt(-d);
       return (double)J;
     };
+    // grid index of tap d < kNcTaps of a point whose first one is q (G >= kNcTaps)
+    auto tap = [](int q, int d, int G) { return q + d < G ? q + d : q + d - G; };
     auto wrap = [](long q, long G) {
       long r = q % G;
       return r < 0 ? r + G : r;
@@ -232,48 +234,57 @@ class NoncartesianOperator : public Operator {
       // row -> (point, tap) over the rows with a weight: a kernel of width 3
       // covers three rows of a point, four only where one is exactly 1.5 away.
       // The partials of the others are never written and stay zero.
-      std::vector<std::vector<int2>> rows(Gy);
+      int *rp = &rptr[(size_t)t * (Gy + 1)];
+      std::vector<int> at(Gy + 1, 0);
       for (long m = 0; m < M; ++m)
         for (int dy = 0; dy < kNcTaps; ++dy)
           if (wyd[m * kNcTaps + dy] != 0.0) {
-            rows[wrap(qy[m] + dy, Gy)].push_back(make_int2((int)m, dy));
+            at[tap(q0[(size_t)t * M + m].y, dy, Gy) + 1]++;
             if (dy == kNcTaps - 1) last[t] = 1;
           }
-      int *rp = &rptr[(size_t)t * (Gy + 1)];
-      for (int r = 0; r < Gy; ++r) {
-        rp[r] = (int)rhdr.size();
-        for (const int2 &md : rows[r]) {
-          const size_t pi = (size_t)t * M + md.x;
-          const float wyd = (&wy4[pi].x)[md.y];
-          rhdr.push_back(make_int4(md.y * (int)M + md.x, r, q0[pi].x, __builtin_bit_cast(int, wyd)));
-          rwx.push_back(wx4[pi]);
-        }
+      at[0] = (int)rhdr.size();
+      for (int r = 0; r < Gy; ++r) at[r + 1] += at[r];
+      std::copy(at.begin(), at.end(), rp);
+      rhdr.resize(rp[Gy]);
+      rwx.resize(rp[Gy]);
+      for (long m = 0; m < M; ++m) {
+        const size_t p = (size_t)t * M + m;
+        for (int dy = 0; dy < kNcTaps; ++dy)
+          if (wyd[m * kNcTaps + dy] != 0.0) {
+            const int r = tap(q0[p].y, dy, Gy), e = at[r]++;
+            const float w = (&wy4[p].x)[dy];
+            rhdr[e] = make_int4(dy * (int)M + (int)m, r, q0[p].x, __builtin_bit_cast(int, w));
+            rwx[e] = wx4[p];
+          }
       }
-      rp[Gy] = (int)rhdr.size();
       // cell -> (point, weight) for the spreading, points in increasing order
       std::vector<int> count(G2, 0);
-      for (long m = 0; m < M; ++m)
+      for (long m = 0; m < M; ++m) {
+        const int2 q = q0[(size_t)t * M + m];
         for (int dy = 0; dy < kNcTaps; ++dy)
           for (int dx = 0; dx < kNcTaps; ++dx)
             if (wyd[m * kNcTaps + dy] * wxd[m * kNcTaps + dx] != 0.0)
-              count[wrap(qy[m] + dy, Gy) * Gx + wrap(qx[m] + dx, Gx)]++;
+              count[(long)tap(q.y, dy, Gy) * Gx + tap(q.x, dx, Gx)]++;
+      }
       int *cp = &cptr[(size_t)t * (G2 + 1)];
       cp[0] = (int)ce.size();
       for (long g = 0; g < G2; ++g) cp[g + 1] = cp[g] + count[g];
       ce.resize(cp[G2]);
       ce_w64.resize(cp[G2]);
       std::vector<int> fill(G2, 0);
-      for (long m = 0; m < M; ++m)
+      for (long m = 0; m < M; ++m) {
+        const int2 q = q0[(size_t)t * M + m];
+        const double sd = std::sqrt((double)dn[(size_t)t * M + m]);
         for (int dy = 0; dy < kNcTaps; ++dy)
           for (int dx = 0; dx < kNcTaps; ++dx) {
             const double w = wyd[m * kNcTaps + dy] * wxd[m * kNcTaps + dx];
             if (w == 0.0) continue;
-            const long cell = wrap(qy[m] + dy, Gy) * Gx + wrap(qx[m] + dx, Gx);
+            const long cell = (long)tap(q.y, dy, Gy) * Gx + tap(q.x, dx, Gx);
             const int pos = cp[cell] + fill[cell]++;
-            const float wf = (float)(w * std::sqrt((double)dn[(size_t)t * M + m]) * sc);
-            ce[pos] = make_int2((int)m, __builtin_bit_cast(int, wf));
-            ce_w64[pos] = w * std::sqrt((double)dn[(size_t)t * M + m]) * sc;
+            ce[pos] = make_int2((int)m, __builtin_bit_cast(int, (float)(w * sd * sc)));
+            ce_w64[pos] = w * sd * sc;
           }
+      }
     }
 
     auto up = [](DevBuf &b, const void *src, size_t bytes) {
