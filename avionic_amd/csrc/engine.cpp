@@ -92,11 +92,12 @@ inline int variant_col_first(int v) { return (v & 1) ? 0 : 1; }
 inline int variant_of(int lanes, bool col_first) { return (lanes == 1 ? 2 : 0) + (col_first ? 0 : 1); }
 // Variant timing (fixed_launch < 0): a launch set is timed once it has run this
 // many plain iterations unchanged, over this many plain iterations per candidate.
-// Measured over 41 launch sets of all methods (64 x 64 to 320 x 300, 1 to 128
-// requests), pairs with the default order are within about 2% of the fastest
-// variant: too little for a timed phase in every launch set by default, which
-// holds the host and two more captures per variant, and during which two runs of
-// tests ended in a host abort whose cause is not established.
+// On the same buffers, from replayed graphs, pairs with the column pass first are
+// within 1.5% of the fastest variant in 18 of 19 launch sets of 16 to 200 requests
+// (64 ICTV 128x128x12x8: one voxel per lane 2.6% faster): too little for a timed
+// phase in every launch set by default, which holds the host and two more captures
+// per variant, and during which two runs of tests ended in a host abort whose
+// cause is not established.
 constexpr int kTuneAfter = 8, kTuneSamples = 3;
 
 // A stream capture and its graph; an exception on the way joins the side stream
@@ -323,14 +324,13 @@ struct avionic_engine {
     // an even width (then both lane variants launch the same kernels); the
     // column pass before or after the dual update (two streams only)
     const int lanes0 = (cfg.voxels_per_lane == 1 || bd2 == 0) ? 1 : 2;
-    const bool first0 = default_col_first(g.grid);
     const bool timing = cfg.fixed_launch < 0;
     g.cands.clear();
     for (int lanes : {2, 1}) {
       if (lanes == 2 && lanes0 == 1) continue;
       if (lanes == 1 && lanes0 == 2 && !timing) continue;
       for (bool first : {true, false}) {
-        if (first != first0 && (!timing || !side)) continue;
+        if (!first && (!timing || !side)) continue;
         g.cands.push_back(variant_of(lanes, first));
       }
     }
@@ -340,7 +340,7 @@ struct avionic_engine {
     auto lg = [](long v) { long k = 0; while (v > 1) { v >>= 1; ++k; } return k; };
     g.sig = {g.method, g.ds, lanes0, lg(g.grid.vox), lg(g.grid.col), lg(g.grid.row), lg(bd1),
              lg(bd2), lg(g.grid.col_groups), wide >= kColWideBlocks};
-    g.variant = variant_of(lanes0, first0);
+    g.variant = variant_of(lanes0, true);
     g.tuning = false;
     g.stable = g.trial = 0;
     for (auto &v : g.samples) v.clear();

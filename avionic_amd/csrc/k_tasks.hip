@@ -96,26 +96,6 @@ const char *kernel_name(int id) {
   return (id >= 0 && id < kNumKernels) ? names[id] : "?";
 }
 
-// Column-pass workgroups up to which the column pass is submitted before the
-// dual: 24 per CU, six waves of the 4 resident per CU (the LDS tile).  Measured
-// on MI355X, dual first against column first: 480 workgroups (ICTGV2
-// 256x256x30x16) +5.7%, 3840 (eight of them) +0.5%, 4800 (twelve TGV2
-// 256x256x25x12) +0.7%, 5520 (with three 192x192x20x10) +1.5%, 5760 (twelve
-// ICTGV2) -0.2%, 6144 (64 TV 128x128x12x8) -0.6%, 7680 (sixteen ICTGV2) -0.1%,
-// 9216 (24 TV 256x256x24x8) -1.0%.
-static int col_first_blocks() {
-  static int n = [] {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
-    return 24 * cus;
-  }();
-  return n;
-}
-
-bool default_col_first(const TaskGrid &gr) { return gr.col <= col_first_blocks(); }
-
 // Dual (primal = false) or primal update over every task, in the grid's
 // launch variant (TaskGrid::lanes).
 template <int M, typename DT, int F>
@@ -194,13 +174,13 @@ void launch_iteration(int method, int ds, const Task *d_tasks, int n, const Task
   const dim3 bRT(RT);
   // dual update (reads ext, writes y) beside the data-term chain (reads ext,
   // writes kcol / z / zhat / khz); the primal update needs both
-  const bool col_first = gr.col_first >= 0 ? gr.col_first == 1 : default_col_first(gr);
-  if (two && col_first) {
-    // The column pass of up to a few waves of workgroups (one reconstruction
-    // of 256x256x30x16: 480 workgroups; eight: 3840) is submitted first, so
-    // that its workgroups start and the dual fills the rest of the CUs; the
-    // dual still depends only on what precedes the column pass.  Larger
-    // column passes go after the dual (default_col_first).
+  if (two && gr.col_first) {
+    // Submitted first, the column pass's workgroups start and the dual fills the
+    // rest of the CUs; the dual still depends only on what precedes the column
+    // pass.  Measured on MI355X, dual first against this order on the same
+    // buffers: 768 column workgroups (16 TV 128x128x12x8) +6% from replayed
+    // graphs, +12% eagerly; 19 sets of 1536 to 12288 workgroups -1.5 to +1.2%
+    // (mean 0) from graphs, 0 to +1.8% eagerly.
     AV_HIP(hipEventRecord(st.fork, s));
     launch_task_col_forward(false, gr, d_tasks, n, s);
     AV_HIP(hipStreamWaitEvent(s2, st.fork, 0));

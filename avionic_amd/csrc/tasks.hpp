@@ -58,9 +58,8 @@ struct TaskGrid {
   int dp1 = 0, dp2 = 0;
   // Launch variant (both give the same bits): lanes 2 runs pairs of voxels
   // for the tasks of even width, lanes 1 one voxel per lane for every task;
-  // col_first 1 submits the column pass before the dual update, 0 after it,
-  // -1 decides by the column pass's grid size.
-  int lanes = 2, col_first = -1;
+  // col_first 1 submits the column pass before the dual update, 0 after it.
+  int lanes = 2, col_first = 1;
   // Blocks [lo, hi) spanning the tasks of each column kind (ColKind) and of
   // each row kind (RowKind); the engine orders its tasks by kind, so each
   // span holds only that kind's blocks.
@@ -87,9 +86,6 @@ struct IterHooks {
 };
 void launch_iteration(int method, int dual_storage, const Task *d_tasks, int n, const TaskGrid &grid,
                       bool with_step, const IterStreams &st, const IterHooks &hooks = IterHooks{});
-// The column-pass order col_first = -1 resolves to: the column pass first
-// when its grid is at most a few waves of workgroups on this device.
-bool default_col_first(const TaskGrid &grid);
 
 // Kernel families of one iteration, in launch order.
 enum KernelId {

@@ -10,7 +10,7 @@
 #include <cstring>
 #include <new>
 #include <string>
-#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/avionic.h"
@@ -192,12 +192,10 @@ size_t first_of(const std::vector<std::string> &v, const char *kernel) {
   CHECK(i < v.size());
   return i;
 }
-// The launch order by the column pass's grid (before the dual update up to 24
-// blocks per CU; the stand-in has 256 CUs), and decisions of their own for launch
-// sets whose row or column grids differ.
+// The column pass is submitted before the dual update in small and large launch
+// sets; sets whose row or column grids differ decide on their variants apart.
 void launch_sets() {
-  for (const auto &[frames, requests, first] :
-       {std::tuple{8u, 1, true}, {128u, 47, true}, {128u, 49, false}}) {
+  for (const auto &[frames, requests] : {std::pair{8u, 1}, {128u, 49}}) {
     avionic_engine *e = engine(config(0, 1));
     std::vector<Req> r;
     for (int i = 0; i < requests; ++i) r.emplace_back(0, frames, 16, 16, 1, 1, 0);
@@ -206,7 +204,7 @@ void launch_sets() {
     stub_take_launches();
     CHECK(avionic_engine_step(e, nullptr) >= 0);
     const std::vector<std::string> v = stub_take_launches();
-    CHECK((first_of(v, "kt_col_forward") < first_of(v, "kt_dual")) == first);
+    CHECK(first_of(v, "kt_col_forward") < first_of(v, "kt_dual"));
     CHECK(avionic_engine_destroy(e) == 0);
   }
   avionic_engine_config c = config(1, 1);
